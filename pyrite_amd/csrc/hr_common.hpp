@@ -59,10 +59,15 @@ __host__ __device__ __forceinline__ uint64_t splitmix64(uint64_t x) {
     return x ^ (x >> 31);
 }
 
-// Draw `counter` of stream `key`, in [0, 1); the 53-bit value converts exactly.
+// The uniform in [0, 1) of one mixed state; the 53-bit value converts exactly.
+__host__ __device__ __forceinline__ double mixed_uniform(uint64_t state) {
+    return (double)(splitmix64(state) >> 11) * kU53;
+}
+
+// Draw `counter` of stream `key`, in [0, 1); draw counter + i is
+// mixed_uniform(state of this one + i kGolden).
 __host__ __device__ __forceinline__ double stream_uniform(uint64_t key, uint64_t counter) {
-    const uint64_t z = splitmix64(key + kGolden * (counter + 1ULL));
-    return (double)(z >> 11) * kU53;
+    return mixed_uniform(key + kGolden * (counter + 1ULL));
 }
 
 // Particle owning compact row r of slot rows laid out by an exclusive prefix

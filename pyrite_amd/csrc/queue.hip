@@ -19,6 +19,9 @@ namespace hr {
 namespace {
 
 constexpr int kQueueMaxCfg = 1024;
+// Configurations whose element constants a block keeps in LDS (52 KB: two
+// 256-lane blocks share a CU's 160 KB); later ones and stacks build them per row.
+constexpr int kQueueEl = 512;
 constexpr int kTally = HR_QUEUE_TALLY;
 
 __device__ __forceinline__ int find_config(const int64_t *__restrict__ off, int n_cfg, int64_t i) {
@@ -55,7 +58,13 @@ __global__ void __launch_bounds__(256) queue_kernel(const hr_queue_config *__res
                                                     double *__restrict__ tally, unsigned long long *next,
                                                     int32_t per_claim) {
     __shared__ int64_t off[kQueueMaxCfg + 1];
+    __shared__ ElConst tab[kQueueEl];
     for (int i = threadIdx.x; i <= n_cfg; i += blockDim.x) off[i] = off_g[i];
+    for (int i = threadIdx.x; i < n_cfg && i < kQueueEl; i += blockDim.x) {
+        const hr_transport_args &t = cfg[i].t;
+        if (t.straggle_on && t.n_layers * t.max_el == 1)
+            tab[i] = make_el(t.L_Z[0], t.L_J[0], t.L_k[0], t.L_coeff[0], t.L_E_cross[0]);
+    }
     __syncthreads();
     Lane s;
     bool live = false, drained = false;
@@ -95,6 +104,8 @@ __global__ void __launch_bounds__(256) queue_kernel(const hr_queue_config *__res
             s.clock = 0.0;
             s.E_cut = q.E_cut_keV;
             s.key = splitmix64(q.seed + kGolden * ((uint64_t)e + 1ULL));
+            s.ukey = splitmix64(s.key ^ kUrbanSalt);
+            s.at.i = -1;
             s.tau = -1.0;
             s.stragg = 0.0;
             s.draws = 0;
@@ -107,7 +118,9 @@ __global__ void __launch_bounds__(256) queue_kernel(const hr_queue_config *__res
         }
         if (__ballot(live || !drained) == 0) break;
         if (live) {
-            const int code = step_lane<false, kMixed>(cfg[c].t, s);
+            const hr_transport_args &t = cfg[c].t;
+            const int n_tab = c < kQueueEl && t.n_layers * t.max_el == 1 ? 1 : 0;
+            const int code = step_lane<false, kMixed>(t, s, tab + (n_tab ? c : 0), n_tab);
             if (code >= 0) {
                 tally_history(tally + (int64_t)c * kTally, s, code, cfg[c].E0_keV);
                 live = false;

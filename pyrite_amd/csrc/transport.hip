@@ -39,17 +39,21 @@ __device__ __forceinline__ int64_t claim(unsigned long long *next, bool want, in
     return id < limit ? id : -1;
 }
 
-// Optional occupancy target (waves per SIMD) for tuning builds; the default
-// lets the compiler keep the whole step in registers.
+// Optional occupancy target (waves per SIMD) for tuning builds.  By default two
+// waves share a SIMD (256 registers each): the plain and continuation kernels
+// hold a step in them, the analytic-law cone kernel spills 28.  The hard-event
+// and tabulated-law cone kernels take one wave and 512.
 #ifdef HR_TRANSPORT_WAVES_PER_EU
-#define HR_TRANSPORT_OCCUPANCY __attribute__((amdgpu_waves_per_eu(HR_TRANSPORT_WAVES_PER_EU, 8)))
+#define HR_TRANSPORT_BOUNDS(two) __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HR_TRANSPORT_WAVES_PER_EU, 8)))
 #else
-#define HR_TRANSPORT_OCCUPANCY
+#define HR_TRANSPORT_BOUNDS(two) __launch_bounds__(256, (two) ? 2 : 1)
 #endif
 
 template <bool kMixed, bool kHard = false, int kCone = 0>
-__global__ void __launch_bounds__(256) HR_TRANSPORT_OCCUPANCY transport_kernel(hr_transport_args a,
+__global__ void HR_TRANSPORT_BOUNDS(!kHard && kCone != 2) transport_kernel(hr_transport_args a,
                                                         unsigned long long *__restrict__ next) {
+    __shared__ ElConst tab[kElSlots];
+    const int n_tab = fill_el_table(a, tab);
     Lane s;
     bool live = false;
     bool drained = false;
@@ -78,13 +82,17 @@ __global__ void __launch_bounds__(256) HR_TRANSPORT_OCCUPANCY transport_kernel(h
             }
         }
         if (__ballot(live || !drained) == 0) break;
-        if (live) {
-            const int code = step_lane<true, kMixed, kHard, kCone>(a, s);
-            if (code >= 0) {
-                store_lane(a, s, (int8_t)code);
-                live = false;
+        // Steps until some lane's electron has ended and it may claim another
+        // (or, once the queue is drained, until every lane's has).
+        do {
+            if (live) {
+                const int code = step_lane<true, kMixed, kHard, kCone>(a, s, tab, n_tab);
+                if (code >= 0) {
+                    store_lane(a, s, (int8_t)code);
+                    live = false;
+                }
             }
-        }
+        } while (__ballot(!live && !drained) == 0 && __ballot(live) != 0);
     }
 }
 
@@ -95,8 +103,10 @@ __global__ void __launch_bounds__(256) HR_TRANSPORT_OCCUPANCY transport_kernel(h
 // accumulator stays in stragg_dE), so a history split over any number of
 // launches emits the rows of one uninterrupted run, bit for bit.
 template <bool kMixed>
-__global__ void __launch_bounds__(256) HR_TRANSPORT_OCCUPANCY continue_kernel(hr_transport_args a,
+__global__ void HR_TRANSPORT_BOUNDS(true) continue_kernel(hr_transport_args a,
                                                                                hr_continuation c) {
+    __shared__ ElConst tab[kElSlots];
+    const int n_tab = fill_el_table(a, tab);
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= a.e_count) return;
     const int64_t h = c.history[i];
@@ -125,7 +135,7 @@ __global__ void __launch_bounds__(256) HR_TRANSPORT_OCCUPANCY continue_kernel(hr
     if (a.max_steps <= 0) {
         code = EXIT_STEP_LIMITED;
     } else {
-        while (code < 0 && s.nseg < a.cap) code = step_lane<true, kMixed>(a, s);
+        while (code < 0 && s.nseg < a.cap) code = step_lane<true, kMixed>(a, s, tab, n_tab);
     }
     store_lane(a, s, code < 0 ? (int8_t)EXIT_SUSPENDED : (int8_t)code);
     c.tau[i] = s.tau;

@@ -13,6 +13,7 @@
 #include "cone.hpp"
 #include "elsepa.hpp"
 #include "hr_common.hpp"
+#include "math64.hpp"
 #include "radiative.hpp"
 #include "shell.hpp"
 
@@ -43,8 +44,8 @@ struct LutPos {
 };
 
 // lut.py:94-110: upper clamp tested first so a non-finite coordinate lands low.
-__device__ __forceinline__ LutPos lut_pos(double E, double log_E_min, double inv_dlogE, int n_energy) {
-    const double x = (log(E) - log_E_min) * inv_dlogE;
+__device__ __forceinline__ LutPos lut_pos(double ln_E, double log_E_min, double inv_dlogE, int n_energy) {
+    const double x = (ln_E - log_E_min) * inv_dlogE;
     const int last = n_energy - 1;
     LutPos p;
     if (x >= (double)last) {
@@ -62,7 +63,7 @@ __device__ __forceinline__ LutPos lut_pos(double E, double log_E_min, double inv
 
 __device__ __forceinline__ double lerp(const double *__restrict__ t, LutPos p) {
     const double lo = t[p.i];
-    return lo + p.f * (t[p.i + 1] - lo);
+    return fma(p.f, t[p.i + 1] - lo, lo);
 }
 
 // Mixed precision (transport/_jit_precision.py:1-40): the table query ln E and
@@ -93,10 +94,13 @@ __device__ __forceinline__ double lerp_f(const float *__restrict__ t, LutPos p) 
 template <bool kMixed>
 struct Lut {
     const hr_transport_args &a;
-    __device__ __forceinline__ LutPos pos(double E) const {
+    // position of energy E, whose logarithm ln_E the FP64 form takes (the mixed
+    // one has its own FP32 query)
+    __device__ __forceinline__ LutPos pos(double E, double ln_E) const {
         return kMixed ? lut_pos_f(E, a.lut_log_E_min, a.lut_inv_dlogE, a.lut_n_energy)
-                      : lut_pos(E, a.lut_log_E_min, a.lut_inv_dlogE, a.lut_n_energy);
+                      : lut_pos(ln_E, a.lut_log_E_min, a.lut_inv_dlogE, a.lut_n_energy);
     }
+    __device__ __forceinline__ LutPos pos(double E) const { return pos(E, kMixed ? 0.0 : ln(E)); }
     __device__ __forceinline__ double rate(size_t off, LutPos p) const {
         return kMixed ? lerp_f(a.lut_total_rate_f + off, p) : lerp(a.lut_total_rate + off, p);
     }
@@ -114,15 +118,58 @@ struct Lut {
     }
 };
 
-// straggling.py:305-329, one element of the spliced stopping, delta = 0.
-__device__ double element_dEds(double J, double k, double coeff, double E_cross, double E) {
-    const double tau = E / kMc2;
-    const double gamma = 1.0 + tau;
-    const double beta_sq = 1.0 - 1.0 / (gamma * gamma);
-    if (E < E_cross) return -7.85e-4 / E * coeff * log(1.166 * (E + k * J) / J);
-    const double f_minus = 1.0 - beta_sq + (tau * tau / 8.0 - (2.0 * tau + 1.0) * kLn2) / (gamma * gamma);
+// What the Urban sampler needs of one element, independent of the energy: five
+// of its logarithms and its exponential.  Kernels build them once per block in
+// LDS; a (layer, element) slot beyond the table is built per row.
+struct ElConst {
+    double J, k, coeff, E_cross;
+    double ln_J, ln_2I2;          // ln J, ln 2 (J / mc^2)^2
+    double e2, ln_e2, f2_e2;      // outer shell: e_2, ln e_2, f_2 / e_2
+    double e1, ln_e1, f1_e1;      // inner level when both shells resolve: e_1, ln e_1, f_1 / e_1
+    double inv_J;
+    double two_shells;            // 1 where Z > 2
+};
+
+__device__ __forceinline__ ElConst make_el(double Z, double J, double k, double coeff, double E_cross) {
+    ElConst c;
+    c.J = J;
+    c.k = k;
+    c.coeff = coeff;
+    c.E_cross = E_cross;
+    c.ln_J = log(J);
     const double I_rel = J / kMc2;
-    return -kBs / beta_sq * coeff * (log(tau * tau * (tau + 2.0) / (2.0 * I_rel * I_rel)) + f_minus - 0.0);
+    c.ln_2I2 = log(2.0 * I_rel * I_rel);
+    c.inv_J = 1.0 / J;
+    c.two_shells = Z > 2.0 ? 1.0 : 0.0;
+    const double f2 = Z > 2.0 ? 2.0 / Z : 1.0;
+    c.e2 = kE2PerZ2 * Z * Z;
+    c.ln_e2 = log(c.e2);
+    c.f2_e2 = f2 / c.e2;
+    c.ln_e1 = c.ln_J;
+    c.e1 = J;
+    c.f1_e1 = c.inv_J;
+    if (Z > 2.0) {
+        const double f1 = 1.0 - f2;
+        c.ln_e1 = (c.ln_J - f2 * c.ln_e2) / f1;
+        c.e1 = exp(c.ln_e1);
+        c.f1_e1 = f1 / c.e1;
+    }
+    return c;
+}
+
+constexpr int kElSlots = 32;  // (layer, element) slots a block keeps in LDS
+
+// Fills a block's table t[kElSlots] and returns its length: every slot of the
+// layer tables, or 0 when there are more than kElSlots (or no straggling).
+__device__ __forceinline__ int fill_el_table(const hr_transport_args &a, ElConst *t) {
+    int n = 0;
+    if (a.straggle_on && (int64_t)a.n_layers * a.max_el <= kElSlots) {
+        n = a.n_layers * a.max_el;
+        for (int i = threadIdx.x; i < n; i += blockDim.x)
+            t[i] = make_el(a.L_Z[i], a.L_J[i], a.L_k[i], a.L_coeff[i], a.L_E_cross[i]);
+    }
+    __syncthreads();
+    return n;
 }
 
 // straggling.py:229-263: inverse-CDF Poisson in bounded chunks, one draw each.
@@ -152,61 +199,147 @@ __device__ int64_t urban_poisson(double lam, uint64_t key, uint64_t &counter) {
     return total;
 }
 
-// straggling.py:131-201 and 278-363: Bragg-additive Urban loss of one layer row.
-__device__ double urban_compound(const double *__restrict__ Zr, const double *__restrict__ Jr,
-                                 const double *__restrict__ kr, const double *__restrict__ cr,
-                                 const double *__restrict__ xr, int n_el, double E, double s,
-                                 uint64_t key) {
+// One term of the three inverse-CDF searches run together.
+struct PoissonTerm {
+    double lam, u, p, cdf;
+    int n;
+    __device__ __forceinline__ void init(double mean, double draw) {
+        lam = mean;
+        u = mean > 0.0 ? draw : -1.0;  // no draw, no events
+        p = exp_neg(mean);
+        cdf = p;
+        n = 0;
+    }
+    __device__ __forceinline__ void next(double inv_k) {
+        n += u >= cdf ? 1 : 0;
+        p = p * (lam * inv_k);
+        cdf = cdf + p;
+    }
+    __device__ __forceinline__ bool open() const { return u >= cdf; }
+};
+
+// The three Poisson numbers of one element (urban_poisson each, in turn).
+// Means of at most one chunk take one draw each, so the three searches step
+// through k together: one chain of three independent recurrences with literal
+// reciprocals instead of three with a division per step.
+__device__ __forceinline__ void urban_counts(double m1, double m2, double m3, uint64_t key, uint64_t &counter,
+                                             int64_t &n1, int64_t &n2, int64_t &n3) {
+    const uint64_t c1 = counter;
+    const uint64_t z1 = key + kGolden * (c1 + 1ULL), z2 = z1 + (m1 > 0.0 ? kGolden : 0ULL);
+    const uint64_t z3 = z2 + (m2 > 0.0 ? kGolden : 0ULL);
+    const double u1 = mixed_uniform(z1), u2 = mixed_uniform(z2), u3 = mixed_uniform(z3);
+    // draws this close to 1 may pass the summed CDF's own rounding: sequential search
+    const double near_one = 1.0 - 1.0e-12;
+    const bool one_chunk = m1 <= kChunk && m2 <= kChunk && m3 <= kChunk && u1 < near_one && u2 < near_one &&
+                           u3 < near_one;
+    if (!one_chunk) {  // also any NaN mean
+        n1 = urban_poisson(m1, key, counter);
+        n2 = urban_poisson(m2, key, counter);
+        n3 = urban_poisson(m3, key, counter);
+        return;
+    }
+    PoissonTerm a, b, c;
+    a.init(m1, u1);
+    b.init(m2, u2);
+    c.init(m3, u3);
+    if (a.open() || b.open() || c.open()) {
+        constexpr double inv[16] = {1.0,     1.0 / 2,  1.0 / 3,  1.0 / 4,  1.0 / 5,  1.0 / 6,  1.0 / 7,  1.0 / 8,
+                                    1.0 / 9, 1.0 / 10, 1.0 / 11, 1.0 / 12, 1.0 / 13, 1.0 / 14, 1.0 / 15, 1.0 / 16};
+        bool open = true;
+#pragma unroll
+        for (int k0 = 0; k0 < 16; k0 += 4) {
+            if (open) {
+#pragma unroll
+                for (int k = k0; k < k0 + 4; ++k) {
+                    a.next(inv[k]);
+                    b.next(inv[k]);
+                    c.next(inv[k]);
+                }
+                open = a.open() || b.open() || c.open();
+            }
+        }
+        for (double k = 17.0; open; k += 1.0) {
+            const double r = rcp_nr(k);
+            a.next(r);
+            b.next(r);
+            c.next(r);
+            open = a.open() || b.open() || c.open();
+        }
+    }
+    n1 = a.n;
+    n2 = b.n;
+    n3 = c.n;
+    counter = c1 + (m1 > 0.0 ? 1ULL : 0ULL) + (m2 > 0.0 ? 1ULL : 0ULL) + (m3 > 0.0 ? 1ULL : 0ULL);
+}
+
+// straggling.py:131-201 and 278-363: Bragg-additive Urban loss of one layer row
+// at energy E (ln_E its logarithm).  The energy enters every logarithm of the
+// model through ln E and ln(tau + 2), taken once per row; the elements' own
+// logarithms come from ElConst.
+__device__ __forceinline__ double urban_compound(const hr_transport_args &a, const ElConst *tab, int n_tab,
+                                                 size_t row, int n_el, double E, double ln_E, double s,
+                                                 uint64_t key) {
     uint64_t counter = 0;
     double loss = 0.0;
-    const double tau = E / kMc2;
+    constexpr double kLnMc2 = 6.236367535407073;   // ln 510.99895
+    constexpr double kLn2Mc2 = 6.929514715967018;  // ln 1021.9979
+    constexpr double kLn50 = 3.912023005428146;    // ln(0.5 / kE0)
+    const double tau = E * (1.0 / kMc2);
     const double gamma = 1.0 + tau;
-    const double beta_sq = 1.0 - 1.0 / (gamma * gamma);
-    const double two = 2.0 * kMc2 * tau * (tau + 2.0);
+    const double inv_g2 = rcp_nr(gamma * gamma);
+    const double beta_sq = tau * (tau + 2.0) * inv_g2;
+    const double ln_tau = ln_E - kLnMc2, ln_tau2 = ln(tau + 2.0);
+    const double ln_t2t2 = 2.0 * ln_tau + ln_tau2;        // ln tau^2 (tau + 2)
+    const double ln_two = kLn2Mc2 + ln_tau + ln_tau2;     // ln 2 mc^2 tau (tau + 2)
+    const double bs = kBs * rcp_nr(beta_sq);
+    const double f_minus = (1.0 + tau * tau * 0.125 - (2.0 * tau + 1.0) * kLn2) * inv_g2;
     const double T_up = 0.5 * E;
+    const double T_w = T_up - kE0, inv_T = rcp_nr(T_up);
+    const double ion = kRate * T_w * inv_T * rcp_nr(kE0 * (ln_E + kLn50));
     for (int el = 0; el < n_el; ++el) {
-        const double Z = Zr[el], J = Jr[el];
-        const double C = -element_dEds(J, kr[el], cr[el], xr[el], E) * 1.0;
+        ElConst q;
+        if (n_tab > 0) {
+            q = tab[row + el];
+        } else {
+            q = make_el(a.L_Z[row + el], a.L_J[row + el], a.L_k[row + el], a.L_coeff[row + el],
+                        a.L_E_cross[row + el]);
+        }
+        // -dE/ds of the element, straggling.py:305-329 (spliced stopping, delta = 0)
+        double C = bs * q.coeff * (ln_t2t2 - q.ln_2I2 + f_minus);
+        if (E < q.E_cross) C = 7.85e-4 / E * q.coeff * log(1.166 * (E + q.k * q.J) / q.J);
         bool valid = T_up > kE0 && C > 0.0;
         double L_I = 0.0;
         if (valid) {
-            L_I = log(two / J) - beta_sq;
+            L_I = ln_two - q.ln_J - beta_sq;
             valid = L_I > 0.0;
         }
         double dE = 0.0;
         if (!valid || !(s > 0.0)) {
             dE = C * s;
         } else {
-            const double e2 = kE2PerZ2 * Z * Z;
-            double f2 = Z > 2.0 ? 2.0 / Z : 1.0;
-            double f1 = 1.0, e1 = J;
-            bool resolved = false;
-            if (Z > 2.0 && e2 < T_up && log(two / e2) - beta_sq > 0.0) {
-                const double f1c = 1.0 - f2;
-                const double e1c = exp((log(J) - f2 * log(e2)) / f1c);
-                if (log(two / e1c) - beta_sq > 0.0) {
-                    f1 = f1c;
-                    e1 = e1c;
-                    resolved = true;
+            const double l2 = ln_two - q.ln_e2 - beta_sq, l1 = ln_two - q.ln_e1 - beta_sq;
+            const bool resolved = q.two_shells != 0.0 && q.e2 < T_up && l2 > 0.0 && l1 > 0.0;
+            const double soft = C * (1.0 - kRate) * rcp_nr(L_I) * s;
+            const double e1 = resolved ? q.e1 : q.J;
+            const double m1 = resolved ? soft * q.f1_e1 * l1 : soft * q.inv_J * L_I;
+            const double m2 = resolved ? soft * q.f2_e2 * l2 : 0.0;
+            int64_t n1, n2, n3;
+            urban_counts(m1, m2, C * ion * s, key, counter, n1, n2, n3);
+            dE = (double)n1 * e1 + (double)n2 * q.e2;
+            // n3 ionisations E_0 / (1 - u (T_up - E_0) / T_up), four draws in flight;
+            // the quotient rounds as the division does, since 1 - quotient cancels
+            // for the rare large transfers
+            uint64_t z = key + kGolden * (counter + 1ULL);
+            counter += (uint64_t)n3;
+            for (int64_t left = n3; left > 0; left -= 4, z += 4ULL * kGolden) {
+                double t[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const double u = mixed_uniform(z + (uint64_t)i * kGolden);
+                    t[i] = kE0 * rcp_nr(1.0 - div_by(u * T_w, T_up, inv_T));
                 }
-            }
-            if (!resolved) {
-                f1 = 1.0;
-                e1 = J;
-                f2 = 0.0;
-            }
-            const double soft = C * (1.0 - kRate) / L_I;
-            const double s1 = soft * (f1 / e1) * (log(two / e1) - beta_sq);
-            const double s2 = f2 > 0.0 ? soft * (f2 / e2) * (log(two / e2) - beta_sq) : 0.0;
-            const double s3 = C * kRate * (T_up - kE0) / (kE0 * T_up * log(T_up / kE0));
-            const int64_t n1 = urban_poisson(s1 * s, key, counter);
-            const int64_t n2 = urban_poisson(s2 * s, key, counter);
-            const int64_t n3 = urban_poisson(s3 * s, key, counter);
-            dE = (double)n1 * e1 + (double)n2 * e2;
-            for (int64_t q = 0; q < n3; ++q) {
-                const double u = stream_uniform(key, counter);
-                counter += 1ULL;
-                dE += kE0 / (1.0 - u * (T_up - kE0) / T_up);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) dE += i < left ? t[i] : 0.0;
             }
         }
         loss += dE;
@@ -219,7 +352,13 @@ __device__ double urban_compound(const double *__restrict__ Zr, const double *__
 // is a lane of the active population).
 struct Lane {
     double px, py, pz, dx, dy, dz, E, clock, tau, E_cut, stragg;
-    uint64_t key, draws;
+    // carried from the end of the previous row while they hold (at.i >= 0): ln E,
+    // the table position of E, and layer `layer`: its faces, element count, and
+    // rate and stopping at E
+    double ln_E, rate, dEds, z_top, z_bot;
+    LutPos at;
+    int layer, n_el;
+    uint64_t key, ukey, draws;  // ukey: the straggling key domain of the history
     int64_t e, id, nseg, flight, substep;
     int32_t steps;
     // hard-event modes: open optical depths (< 0: draw at the next step), keys, counters
@@ -242,6 +381,8 @@ __device__ __forceinline__ void load_lane(const hr_transport_args &a, int64_t e,
     s.clock = a.clock[e];
     s.E_cut = a.E_cut[e];
     s.key = a.stream_key[e];
+    s.ukey = splitmix64(s.key ^ kUrbanSalt);
+    s.at.i = -1;
     s.tau = -1.0;
     s.stragg = 0.0;
     s.draws = 0;
@@ -291,26 +432,25 @@ __device__ __forceinline__ void rotate_lane(Lane &s, double cos_t, double phi) {
         sin_phi = (double)sf;
         cos_phi = (double)cf;
     } else {
-        sin_t = sqrt(s2 > 0.0 ? s2 : 0.0);
-        sin_phi = sin(phi);
-        cos_phi = cos(phi);
+        sin_t = s2 > 0.0 ? s2 * rsqrt_nr(s2) : 0.0;
+        sincos_phi(phi, sin_phi, cos_phi);
     }
     double refx, refy;
     if (fabs(dx) < 0.9) { refx = 1.0; refy = 0.0; } else { refx = 0.0; refy = 1.0; }
     double ux = -dz * refy, uy = dz * refx, uz = dx * refy - dy * refx;
-    const double u_mag = sqrt(ux * ux + uy * uy + uz * uz);
-    ux = ux / u_mag;
-    uy = uy / u_mag;
-    uz = uz / u_mag;
+    const double inv_u = rsqrt_nr(fma(uz, uz, fma(uy, uy, ux * ux)));
+    ux = ux * inv_u;
+    uy = uy * inv_u;
+    uz = uz * inv_u;
     const double wx = dy * uz - dz * uy, wy = dz * ux - dx * uz, wz = dx * uy - dy * ux;
     const double ra = sin_t * cos_phi, rb = sin_t * sin_phi;
-    const double ox = cos_t * dx + ra * ux + rb * wx;
-    const double oy = cos_t * dy + ra * uy + rb * wy;
-    const double oz = cos_t * dz + ra * uz + rb * wz;
-    const double mag = sqrt(ox * ox + oy * oy + oz * oz);
-    s.dx = ox / mag;
-    s.dy = oy / mag;
-    s.dz = oz / mag;
+    const double ox = fma(rb, wx, fma(ra, ux, cos_t * dx));
+    const double oy = fma(rb, wy, fma(ra, uy, cos_t * dy));
+    const double oz = fma(rb, wz, fma(ra, uz, cos_t * dz));
+    const double inv_o = rsqrt_nr(fma(oz, oz, fma(oy, oy, ox * ox)));
+    s.dx = ox * inv_o;
+    s.dy = oy * inv_o;
+    s.dz = oz * inv_o;
 }
 
 __device__ __forceinline__ void store_lane(const hr_transport_args &a, const Lane &s, int8_t code) {
@@ -337,8 +477,9 @@ __device__ __forceinline__ void store_lane(const hr_transport_args &a, const Lan
 // kCone: 0 no splitting; 1 copies on the screened-Rutherford law; 2 copies on
 // the tabulated (ELSEPA) law, a variant of its own so the bisection's
 // registers stay out of the other kernels.
+// tab holds the element constants of the first n_tab (layer, element) slots.
 template <bool kRows = true, bool kMixed = false, bool kHard = false, int kCone = 0>
-__device__ int step_lane(const hr_transport_args &a, Lane &s) {
+__device__ int step_lane(const hr_transport_args &a, Lane &s, const ElConst *tab, int n_tab) {
     const Lut<kMixed> lut{a};
     const int nE = a.lut_n_energy;
     const int max_el = a.max_el;
@@ -352,15 +493,29 @@ __device__ int step_lane(const hr_transport_args &a, Lane &s) {
         }
         L = lo;
     }
-    const int n_el = a.L_nel[L];
-    const double z_top = a.L_top[L], z_bot = a.L_bot[L];
     const double E = s.E;
-    const LutPos p = lut.pos(E);
     const size_t row_off = (size_t)L * nE;
-    const double total_rate = lut.rate(row_off, p);
-    const double lam = 1e8 / total_rate;
+    if (s.at.i < 0) {
+        s.ln_E = ln(E);
+        s.at = lut.pos(E, s.ln_E);
+        s.layer = -1;
+    }
+    const LutPos p = s.at;
+    const double ln_E = s.ln_E;
+    if (s.layer != L) {
+        s.n_el = a.L_nel[L];
+        s.z_top = a.L_top[L];
+        s.z_bot = a.L_bot[L];
+        s.rate = lut.rate(row_off, p);
+        s.dEds = lut.dEds(row_off, p);
+    }
+    const int n_el = s.n_el;
+    const double z_top = s.z_top, z_bot = s.z_bot;
+    const double total_rate = s.rate, dEds_j = s.dEds;
+    const double lam = 1e8 * rcp_nr(total_rate);
     if (s.tau < 0.0) {
-        s.tau = -log(stream_uniform(s.key, s.draws));
+        const double u = stream_uniform(s.key, s.draws);
+        s.tau = u > 0.0 ? -ln(u) : INFINITY;
         s.draws += 1ULL;
     }
     double step = s.tau * lam;
@@ -415,24 +570,23 @@ __device__ int step_lane(const hr_transport_args &a, Lane &s) {
             side = face >= 0 && face <= 3;
         }
     } else if (dz < 0.0) {
-        const double sb = (pz - z_top) / (-dz);
+        const double sb = (z_top - pz) * rcp_nr(dz);
         if (step > sb) { step = sb; up = true; }
     } else if (dz > 0.0) {
-        const double sb = (z_bot - pz) / dz;
+        const double sb = (z_bot - pz) * rcp_nr(dz);
         if (step > sb) { step = sb; dn = true; }
     }
     bool exit_top = up && z_top <= 0.0;
     bool exit_bot = dn && z_bot >= a.z_total;
     // soft radiative stopping joins the collision stopping as a mean loss
-    const double dEds = kHard ? lut.dEds(row_off, p) - rad_dEds : lut.dEds(row_off, p);
-    const double inv_beta_j = lut.inv_beta(p);
+    const double dEds = kHard ? dEds_j - rad_dEds : dEds_j;
     bool cutoff = false, limited = false;
     bool geometry_event = up || dn || side;
     double E_end, t_end;
     const bool midpoint = a.energy_model == 1;
     if (a.straggle_on) {
         if (a.max_dE_frac > 0.0) {
-            const double se = a.max_dE_frac * E / (-dEds);
+            const double se = a.max_dE_frac * E * rcp_nr(-dEds);
             if (se < step) {
                 step = se;
                 limited = true;
@@ -440,9 +594,8 @@ __device__ int step_lane(const hr_transport_args &a, Lane &s) {
                 geometry_event = false;
             }
         }
-        const uint64_t ukey = splitmix64(s.key ^ kUrbanSalt);
         const uint64_t combined = ((uint64_t)s.flight << 32) + (uint64_t)s.substep;
-        const uint64_t fkey = splitmix64(ukey + kGolden * combined);
+        const uint64_t fkey = splitmix64(s.ukey + kGolden * combined);
         const size_t row = (size_t)L * max_el;
         double loss;
         if (kHard && a.hard.shell_on) {
@@ -451,8 +604,7 @@ __device__ int step_lane(const hr_transport_args &a, Lane &s) {
             uint64_t counter = 0;
             loss = shell::soft_loss(-(dEds + rad_dEds) * step, omega2 * step, fkey, counter);
         } else {
-            loss = urban_compound(a.L_Z + row, a.L_J + row, a.L_k + row, a.L_coeff + row, a.L_E_cross + row,
-                                  n_el, E, step, fkey);
+            loss = urban_compound(a, tab, n_tab, row, n_el, E, ln_E, step, fkey);
         }
         if (kHard) loss += rad_dEds * step;
         s.stragg += loss;
@@ -470,7 +622,7 @@ __device__ int step_lane(const hr_transport_args &a, Lane &s) {
             const LutPos c = lut.pos(0.5 * (E + E_end));
             t_end = s.clock + step * lut.inv_beta(c);
         } else {
-            t_end = s.clock + step * inv_beta_j;
+            t_end = s.clock + step * lut.inv_beta(p);
         }
     } else {
         double cut_dist;
@@ -509,9 +661,15 @@ __device__ int step_lane(const hr_transport_args &a, Lane &s) {
             t_end = s.clock + step * lut.inv_beta(c);
         } else {
             E_end = cutoff ? s.E_cut : E + dEds * step;
-            t_end = s.clock + step * inv_beta_j;
+            t_end = s.clock + step * lut.inv_beta(p);
         }
     }
+    // Table values of the row's end: the next row's start, and the screening of
+    // the collision there.  They are read before the row is stored, because a
+    // load waits for every store issued before it.
+    const double ln_end = (!kMixed || a.straggle_on) ? ln(E_end) : 0.0;
+    const LutPos pe = lut.pos(E_end, ln_end);
+    const double rate_end = lut.rate(row_off, pe), dEds_end = lut.dEds(row_off, pe);
     int8_t event = EV_ELASTIC;
     if (limited) event = EV_SUBSTEP;
     else if (cutoff) event = EV_CUTOFF;
@@ -594,14 +752,38 @@ __device__ int step_lane(const hr_transport_args &a, Lane &s) {
         }
     }
 
+    // Elastic collision: element (cores.py:1094-1105), screened-Rutherford angle.
+    const size_t el_row = (size_t)L * max_el;
+    int i_el = 0;
+    double cos_u = 0.0, phi_u = 0.0, alpha = 0.0;
+    if (event == EV_ELASTIC) {
+        if (n_el != 1) {
+            const double u = stream_uniform(s.key, s.draws);
+            s.draws += 1ULL;
+            i_el = n_el - 1;
+            for (int k = 0; k < n_el; ++k) {
+                if (lut.cdf((el_row + k) * nE, p) > u) {
+                    i_el = k;
+                    break;
+                }
+            }
+        }
+        if (!a.elsepa.on) alpha = lut.alpha((el_row + i_el) * nE, pe);
+        const uint64_t z = s.key + kGolden * (s.draws + 1ULL);
+        cos_u = mixed_uniform(z);
+        phi_u = mixed_uniform(z + kGolden);
+        s.draws += 2ULL;
+    }
+
     if (kRows && s.nseg < a.cap) {
         const int64_t slot = (s.e - a.e_start) * a.cap + s.nseg;
         a.seg_dir[3 * slot] = dx;
         a.seg_dir[3 * slot + 1] = dy;
         a.seg_dir[3 * slot + 2] = dz;
-        a.seg_mid[3 * slot] = px + 0.5 * step * dx;
-        a.seg_mid[3 * slot + 1] = py + 0.5 * step * dy;
-        a.seg_mid[3 * slot + 2] = pz + 0.5 * step * dz;
+        const double half = 0.5 * step;
+        a.seg_mid[3 * slot] = fma(half, dx, px);
+        a.seg_mid[3 * slot + 1] = fma(half, dy, py);
+        a.seg_mid[3 * slot + 2] = fma(half, dz, pz);
         a.seg_len[slot] = step;
         a.seg_E[slot] = E;
         a.seg_t0[slot] = s.clock;
@@ -626,12 +808,17 @@ __device__ int step_lane(const hr_transport_args &a, Lane &s) {
         }
     }
     s.nseg += 1;
-    s.px = px + step * dx;
-    s.py = py + step * dy;
-    s.pz = pz + step * dz;
+    s.px = fma(step, dx, px);
+    s.py = fma(step, dy, py);
+    s.pz = fma(step, dz, pz);
     s.E = E_end;
+    s.ln_E = ln_end;
+    s.at = pe;
+    s.layer = L;
+    s.rate = rate_end;
+    s.dEds = dEds_end;
     s.clock = t_end;
-    s.tau -= step / lam;
+    s.tau -= step * total_rate * 1e-8;
     if (s.tau < 0.0) s.tau = 0.0;
     if constexpr (kHard) {
         if (a.hard.shell_on) {
@@ -665,39 +852,24 @@ __device__ int step_lane(const hr_transport_args &a, Lane &s) {
     if constexpr (kHard) {
         if (event == EV_HARD_RADIATIVE) {  // debit the photon; no deflection, no elastic draw
             s.E -= rad_k * 1.0e-3;
+            s.at.i = -1;
             s.steps += 1;
             return s.steps < a.max_steps ? -1 : EXIT_STEP_LIMITED;
         }
         if (event == EV_HARD_INELASTIC) {  // the loss and recoil deflection replace the elastic draw
             s.E -= hard_W;
+            s.at.i = -1;
             rotate_lane<kMixed>(s, hard_cos, hard_phi);
             s.steps += 1;
             return s.steps < a.max_steps ? -1 : EXIT_STEP_LIMITED;
         }
     }
-    // Elastic collision: element (cores.py:1094-1105), screened-Rutherford angle.
-    const size_t el_row = (size_t)L * max_el;
-    int i_el = 0;
-    if (n_el != 1) {
-        const double u = stream_uniform(s.key, s.draws);
-        s.draws += 1ULL;
-        i_el = n_el - 1;
-        for (int k = 0; k < n_el; ++k) {
-            if (lut.cdf((el_row + k) * nE, p) > u) {
-                i_el = k;
-                break;
-            }
-        }
-    }
-    const double cos_u = stream_uniform(s.key, s.draws);
-    const double phi_u = stream_uniform(s.key, s.draws + 1ULL);
-    s.draws += 2ULL;
-    double alpha = 0.0, cos_t;
+    double cos_t;
     if (a.elsepa.on) {  // tabulated angles at the same uniform (_jit_kernel.py:1149-1160)
         cos_t = 1.0 - 2.0 * elsepa::sample_mu(a.elsepa, el_row + i_el, s.E, cos_u);
     } else {
-        alpha = lut.alpha((el_row + i_el) * nE, lut.pos(s.E));
-        cos_t = 1.0 - 2.0 * alpha * cos_u / (1.0 + alpha - cos_u);
+        const double den = 1.0 + alpha - cos_u;
+        cos_t = 1.0 - div_by(2.0 * alpha * cos_u, den, rcp_nr(den));
     }
     bool split_here = false;
     if constexpr (kCone != 0) {

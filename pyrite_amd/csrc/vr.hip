@@ -33,6 +33,8 @@ __host__ __device__ __forceinline__ uint64_t child_key(uint64_t key, int64_t j) 
 template <bool kMixed>
 __global__ void __launch_bounds__(256) vr_round_kernel(hr_transport_args a, int32_t rows,
                                                        const int32_t *__restrict__ rows_each) {
+    __shared__ ElConst tab[kElSlots];
+    const int n_tab = fill_el_table(a, tab);
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= a.e_count) return;
     const int64_t e = a.e_start + i;
@@ -44,7 +46,7 @@ __global__ void __launch_bounds__(256) vr_round_kernel(hr_transport_args a, int3
     Lane s;
     load_lane(a, e, s);
     int code = -1;
-    while (code < 0 && s.nseg < mine) code = step_lane<true, kMixed>(a, s);
+    while (code < 0 && s.nseg < mine) code = step_lane<true, kMixed>(a, s, tab, n_tab);
     store_lane(a, s, code < 0 ? (int8_t)EXIT_SUSPENDED : (int8_t)code);
 }
 
