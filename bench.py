@@ -559,7 +559,7 @@ def main():
             "parallelism": "single GPU",
         },
         "roofline": {
-            "kernel": "hr_sincsq_reduce: sincsq_uniform_kernel + sum_partials_kernel (dense sinc^2 lines)",
+            "kernel": "hr_sincsq_reduce: sincsq_uniform_kernel + row_sum_kernel (dense sinc^2 lines)",
             "bound": "valu",
             "pipe": "vector ALU, FP32 peak (the listed fp32 dense figure equals the VALU FP32 peak)",
             "achieved": achieved,

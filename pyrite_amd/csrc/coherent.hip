@@ -25,6 +25,7 @@
 
 #include "hr_common.hpp"
 #include "line_core.hpp"
+#include "row_sum.hpp"
 
 namespace hr {
 namespace {
@@ -348,16 +349,6 @@ __global__ void __launch_bounds__(kFieldThreads) coherent_grouped_kernel(hr_cohe
     }
 }
 
-// field[i] += sum_s partial[s][i] in split order, i over n_rows*4*n_E cells.
-__global__ void __launch_bounds__(256) field_partials_kernel(const double *__restrict__ partial, int S,
-                                                             int64_t cells, double *__restrict__ field) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= cells) return;
-    double s = 0.0;
-    for (int k = 0; k < S; ++k) s += partial[(int64_t)k * cells + i];
-    field[i] += s;
-}
-
 __global__ void __launch_bounds__(256) coherent_finalize_kernel(const double *__restrict__ field, int n_dir, int n_g,
                                                                 const double *__restrict__ dir_weight,
                                                                 const double *__restrict__ wm, int64_t n_E,
@@ -523,12 +514,7 @@ extern "C" hr_status hr_coherent_field(const hr_coherent_field_args *args, void 
     hipLaunchKernelGGL(coherent_field_kernel<kFieldBins>, dim3((unsigned)S, (unsigned)(p.n_rows * W)),
                        dim3(kFieldThreads), 0, s, p, (int)W, (int)S, out);
     HR_CHECK_HIP(hipGetLastError());
-    if (S > 1) {
-        hipLaunchKernelGGL(field_partials_kernel, dim3((unsigned)blocks_of(cells, 256)), dim3(256), 0, s,
-                           (const double *)ws, (int)S, cells, p.field);
-        HR_CHECK_HIP(hipGetLastError());
-    }
-    return HR_OK;
+    return S > 1 ? row_sum((const double *)ws, S, cells, p.field, s) : HR_OK;
 }
 
 extern "C" hr_status hr_coherent_finalize(const double *field, int32_t n_dir, int32_t n_g, const double *dir_weight,
@@ -583,12 +569,7 @@ extern "C" hr_status hr_coherent_grouped(const hr_coherent_grouped_args *args, v
     hipLaunchKernelGGL(coherent_grouped_kernel<kFieldBins>, dim3((unsigned)S, (unsigned)(p.n_rows * W)),
                        dim3(kFieldThreads), 0, s, p, args->group_start, n_groups, (int)W, (int)S, out);
     HR_CHECK_HIP(hipGetLastError());
-    if (S > 1) {
-        hipLaunchKernelGGL(field_partials_kernel, dim3((unsigned)blocks_of(cells, 256)), dim3(256), 0, s,
-                           (const double *)p.ws.ptr, (int)S, cells, args->grouped);
-        HR_CHECK_HIP(hipGetLastError());
-    }
-    return HR_OK;
+    return S > 1 ? row_sum((const double *)p.ws.ptr, S, cells, args->grouped, s) : HR_OK;
 }
 
 extern "C" hr_status hr_coherent_blend_finalize(const double *field, const double *grouped, int32_t n_dir,

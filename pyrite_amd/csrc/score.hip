@@ -23,6 +23,7 @@
 
 #include "hr_common.hpp"
 #include "line_core.hpp"
+#include "row_sum.hpp"
 
 namespace hr {
 namespace {
@@ -232,35 +233,6 @@ __global__ void __launch_bounds__(kRedThreads) sincsq_general_kernel(
         if (k < n_E) out[k] = acc[m];
     }
 }
-
-// out[k] += sum_b partial[b][k], b ascending (fixed order).
-__global__ void __launch_bounds__(256) sum_partials_kernel(const double *__restrict__ partial,
-                                                           int64_t n_part, int64_t n_E,
-                                                           double *__restrict__ out) {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n_E) return;
-    double s = 0.0;
-    for (int64_t b = 0; b < n_part; ++b) s += partial[b * n_E + k];
-    out[k] += s;
-}
-
-// First level of the fixed-order partial sum: split s adds rows
-// [s*chunk, min((s+1)*chunk, n_part)) of every bin into level[s][k].
-__global__ void __launch_bounds__(256) sum_partials_split_kernel(const double *__restrict__ partial,
-                                                                 int64_t n_part, int64_t chunk, int64_t n_E,
-                                                                 double *__restrict__ level) {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n_E) return;
-    const int64_t b0 = (int64_t)blockIdx.y * chunk;
-    const int64_t b1 = b0 + chunk < n_part ? b0 + chunk : n_part;
-    double s = 0.0;
-    for (int64_t b = b0; b < b1; ++b) s += partial[b * n_E + k];
-    level[(int64_t)blockIdx.y * n_E + k] = s;
-}
-
-// Splits of the two-level partial sum (a fixed tree: deterministic, and wide
-// enough that the first level reads the partials at full bandwidth).
-constexpr int64_t kPartialSplits = 64;
 
 constexpr float kMc2f = 510.99895f;
 constexpr float kInvMc2f = (float)(1.0 / 510.99895);
@@ -628,26 +600,8 @@ __global__ void fill_zero_kernel(double *__restrict__ p, int64_t n) {
     if (i < n) p[i] = 0.0;
 }
 
-// Workspace bytes for gx partial rows of n_E bins plus the second level.
-size_t partial_bytes(int64_t gx, int64_t n_E) {
-    const int64_t splits = gx < kPartialSplits ? gx : kPartialSplits;
-    return (size_t)(gx + splits) * (size_t)n_E * sizeof(double);
-}
-
-// out[k] += the fixed two-level sum of gx partial rows held at ws.
-hr_status reduce_partials(void *ws, int64_t gx, int64_t n_E, double *out, hipStream_t s) {
-    const double *partial = (const double *)ws;
-    const int64_t splits = gx < kPartialSplits ? gx : kPartialSplits;
-    const int64_t chunk = (gx + splits - 1) / splits;
-    double *level = (double *)ws + gx * n_E;
-    const unsigned bx = (unsigned)((n_E + 255) / 256);
-    hipLaunchKernelGGL(sum_partials_split_kernel, dim3(bx, (unsigned)splits), dim3(256), 0, s, partial, gx, chunk,
-                       n_E, level);
-    HR_CHECK_HIP(hipGetLastError());
-    hipLaunchKernelGGL(sum_partials_kernel, dim3(bx), dim3(256), 0, s, (const double *)level, splits, n_E, out);
-    HR_CHECK_HIP(hipGetLastError());
-    return HR_OK;
-}
+// Workspace bytes for gx partial rows of n_E bins.
+size_t partial_bytes(int64_t gx, int64_t n_E) { return (size_t)gx * (size_t)n_E * sizeof(double); }
 
 // Blocks along the line axis: enough to fill the chip several times over, but
 // never more than there are line tiles.
@@ -744,7 +698,7 @@ extern "C" hr_status hr_sincsq_reduce(const hr_sincsq_args *args, void *stream) 
                            p.n_lines, p.E_grid, p.n_E, (double *)ws);
     }
     HR_CHECK_HIP(hipGetLastError());
-    return reduce_partials(ws, gx, p.n_E, p.out, s);
+    return row_sum((const double *)ws, gx, p.n_E, p.out, s);
 }
 
 // Scratch of hr_sincsq_reduce_static: the partial spectra of one call live in
@@ -784,10 +738,12 @@ extern "C" hr_status hr_sincsq_reduce_static(const hr_sincsq_args *args, void *s
     DensePlan P;
     hr_status st = dense_plan(args->n_lines, kLineTile, args->n_E, P);
     if (st != HR_OK) return st;
-    HR_REQUIRE(P.bytes <= (size_t)HR_SINCSQ_STATIC_SCRATCH_BYTES,
+    // the sizes taken are those whose partials and 64 rows more fit
+    const size_t need = partial_bytes(P.gx + (P.gx < 64 ? P.gx : 64), args->n_E);
+    HR_REQUIRE(need <= (size_t)HR_SINCSQ_STATIC_SCRATCH_BYTES,
                "hr_sincsq_reduce_static: %lld bins need %zu bytes of partials, more than the %zu-byte static "
                "scratch (use hr_sincsq_reduce with a workspace)",
-               (long long)args->n_E, P.bytes, (size_t)HR_SINCSQ_STATIC_SCRATCH_BYTES);
+               (long long)args->n_E, need, (size_t)HR_SINCSQ_STATIC_SCRATCH_BYTES);
     void *ptr = nullptr;
     st = static_scratch(&ptr);
     if (st != HR_OK) return st;
@@ -845,7 +801,7 @@ extern "C" hr_status hr_brem_reduce(const hr_brem_args *args, void *stream) {
     default: hipLaunchKernelGGL((brem_kernel<BINS, 4>), grid, dim3(kRedThreads), 0, s, p, (double *)ws); break;
     }
     HR_CHECK_HIP(hipGetLastError());
-    return reduce_partials(ws, gx, p.n_E, p.out, s);
+    return row_sum((const double *)ws, gx, p.n_E, p.out, s);
 }
 
 namespace hr {
