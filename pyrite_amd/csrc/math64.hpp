@@ -36,6 +36,9 @@ __device__ __forceinline__ double rsqrt_nr(double x) {
     return fma(fma(-h * r, r, 0.5), r, r);
 }
 
+// sqrt(x) for x > 0 (a negative or NaN x gives NaN).
+__device__ __forceinline__ double sqrt_nr(double x) { return x * rsqrt_nr(x); }
+
 // ln x for finite x > 0 (a NaN stays one): k ln 2 + 2 atanh(s), s = (m - 1)/(m + 1),
 // m in [sqrt(1/2), sqrt(2)), the series of atanh to s^23 (|s| <= 0.1716:
 // remainder below 1e-18).
@@ -57,11 +60,11 @@ __device__ __forceinline__ double ln(double x) {
     return fma(e, kLn2Hi, fma(s, 2.0, fma(s * z, P, e * kLn2Lo)));
 }
 
-// exp(-x) for 0 <= x <= 64: 2^k times the Taylor series to r^13 on |r| <= ln(2)/2
-// (remainder below 1e-16).
-__device__ __forceinline__ double exp_neg(double x) {
-    const double k = rint(x * -1.4426950408889634);
-    const double r = fma(k, -kLn2Lo, fma(k, -kLn2Hi, -x));
+// exp(x) for finite x: 2^k times the Taylor series to r^13 on |r| <= ln(2)/2
+// (remainder below 1e-16); far negative arguments underflow to zero.
+__device__ __forceinline__ double exp_any(double x) {
+    const double k = rint(x * 1.4426950408889634);
+    const double r = fma(k, -kLn2Lo, fma(k, -kLn2Hi, x));
     const double r2 = r * r, r4 = r2 * r2;
     const double a0 = fma(r, 1.0 / 6, 0.5), a1 = fma(r, 1.0 / 120, 1.0 / 24), a2 = fma(r, 1.0 / 5040, 1.0 / 720);
     const double a3 = fma(r, 1.0 / 362880, 1.0 / 40320), a4 = fma(r, 1.0 / 39916800, 1.0 / 3628800);

@@ -23,6 +23,7 @@
 
 #include "hr_common.hpp"
 #include "line_core.hpp"
+#include "math64.hpp"
 #include "row_sum.hpp"
 
 namespace hr {
@@ -106,85 +107,174 @@ constexpr int kRedThreads = 256;
 constexpr int kLineTile = 256;  // lines staged in LDS per step
 constexpr int kSincGroup = 4;   // cells summed in FP32 before each FP64 add (all terms >= 0)
 
-// Dense sum over a uniform grid E_k = E0 + k dE.  Block b takes line tiles
-// b, b + gridDim.x, ...; thread t owns bins t + kRedThreads*m (m < BINS_PER_THREAD)
-// of the bin window starting at blockIdx.y * kRedThreads * BINS.  A staged line
-// is (u0, du) in one 16-byte LDS slot (one ds_read_b128) with the weights of
-// kSincGroup lines in one float4; a group whose lines all have zero weight
-// (copies that do not carry this tally) costs one LDS read.  The phase
-// u = u0 + k du is formed and reduced in FP64 per cell: on this device an FP64
-// FMA/add issues at the rate of a non-packed FP32 one, and FP32 stepping of the
-// reduced phase would take more instructions per cell.
-template <int BINS>
-__global__ void __launch_bounds__(kRedThreads) sincsq_uniform_kernel(
-    const double *__restrict__ E_r, const double *__restrict__ a, const float *__restrict__ w,
-    int64_t n_lines, double E0, double dE, int64_t n_E, double *__restrict__ partial) {
-    static_assert(kSincGroup == 4 && kLineTile % kSincGroup == 0, "weights are read as float4 groups");
-    __shared__ double2 s_ud[kLineTile];
-    __shared__ float4 s_w4[kLineTile / kSincGroup];
-    float *s_w = reinterpret_cast<float *>(s_w4);
-    const int t = threadIdx.x;
-    const int64_t bin0 = (int64_t)blockIdx.y * kRedThreads * BINS;
-    double acc[BINS], kd[BINS];
+// ---- dense sum over a uniform grid E_k = E0 + k dE
+//
+// A line's profile is w sin^2(pi u)/(pi u)^2 with u = u0 + k du, so along a run of
+// bins sin(pi u) obeys s[k+1] = 2 cos(pi du) s[k] - s[k-1]: one FP64 FMA per
+// cell instead of a phase, its reduction and a polynomial.  A wave owns a window
+// of 64 BINS bins, BINS consecutive ones per lane; per line each lane takes one
+// sine and cosine at the middle of its run and steps outward both ways (at most
+// BINS/2 steps: the sines stay within 1e-13).  The divisor is the distance in
+// bins, d = (k - n) + u(n)/du with n the bin nearest the centre, so it is exact to
+// FP32 rounding there; sqrt(w)/(pi du) rides on the sines.
+//
+// VALU bound: about 31 SIMD cycles per cell (FP64, conversions and selects issue
+// in 4, plain FP32 in 2, the reciprocal in 8) against 52 of a cell with its own
+// phase.  2.7e6 lines (half live) on 1024 bins: 608 us before, 402 now
+// (about 49 cycles: staging, FP64 sums and waves of uneven work make the rest).
+constexpr int kSincWaves = 4;     // waves per block, each with its own lines
+constexpr int kSincBlock = 64 * kSincWaves;
+constexpr int kSincChunk = 64;    // lines a wave stages at a time (one per lane)
+
+// sin(pi r)/r and cos(pi r) on |r| <= 1/2 in r^2 (Chebyshev interpolation of
+// each; errors 1.6e-13 and 2.0e-15).
+constexpr double kSinR[7] = {3.141592653589635, -5.167712779987959, 2.550164035906745, -0.5992644339357286, 0.08214479467064854,
+          -0.007364005472115722, 0.0004474920849077101};
+constexpr double kCosR[8] = {0.9999999999999981, -4.934802200543686, 4.058712126333295, -1.3352627661817635, 0.23533058831317874,
+          -0.025806531975921563, 0.0019278700526981333, -0.0001004164642205389};
+
+template <int N>
+__device__ __forceinline__ double horner(const double (&c)[N], double z) {
+    double p = c[N - 1];
 #pragma unroll
-    for (int m = 0; m < BINS; ++m) {
-        acc[m] = 0.0;
-        kd[m] = (double)(bin0 + t + (int64_t)m * kRedThreads);
+    for (int i = N - 2; i >= 0; --i) p = fma(p, z, c[i]);
+    return p;
+}
+
+// A staged live line.
+struct alignas(16) SincLine {
+    double u0, du;    // u = u0 + k du, turns of pi
+    double cd, sd;    // cos, sin of pi du
+    double q;         // sqrt(w) / (pi du)
+    float nf, f, w;   // n - bin0 for the integer n nearest the centre; u(n)/du; w
+    int direct;       // no recurrence: see the staging
+};
+
+template <int BINS>
+__global__ void __launch_bounds__(kSincBlock, 4) sincsq_uniform_kernel(
+    const double *__restrict__ E_r, const double *__restrict__ a, const float *__restrict__ w, int64_t n_lines,
+    int per, double E0, double dE, int64_t n_E, double *__restrict__ partial) {
+    static_assert(BINS % 4 == 0 && BINS >= 4, "runs are stepped outward from their middle");
+    constexpr int kWindow = 64 * BINS, kMid = BINS / 2;
+    __shared__ SincLine s_line[kSincWaves][kSincChunk];
+    __shared__ double s_sum[kWindow];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t bin0 = (int64_t)blockIdx.y * kWindow;
+    const int run0 = lane * BINS;                           // first bin of the lane's run, from bin0
+    const double kb = (double)(bin0 + run0 + kMid);         // its middle
+    const float run0f = (float)run0;
+    SincLine *lines = s_line[wave];
+    double acc[BINS];
+#pragma unroll
+    for (int m = 0; m < BINS; ++m) acc[m] = 0.0;
+    const double inv_pi = 1.0 / kPi, inv_dE = 1.0 / dE;
+    // the coefficients in scalar registers, from which an FMA reads them directly
+    double sin_r[7], cos_r[8];
+#pragma unroll
+    for (int i = 0; i < 7; ++i) {
+        sin_r[i] = kSinR[i];
+        asm volatile("" : "+s"(sin_r[i]));
     }
-    const double inv_pi = 1.0 / kPi;
-    const int64_t n_tiles = (n_lines + kLineTile - 1) / kLineTile;
-    for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-        const int64_t l = tile * kLineTile + t;
-        // u(E_k) = a (E_k - E_r)/pi = u0 + k du; the weight is read first and a
-        // zero-weight line's E_r and a are never fetched (rejected resonances
-        // come in whole waves: a ray whose in-medium root never settles)
-        const float wl = l < n_lines ? w[l] : 0.0f;
-        s_w[t] = wl;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        cos_r[i] = kCosR[i];
+        asm volatile("" : "+s"(cos_r[i]));
+    }
+    const int64_t n_chunks = (n_lines + per - 1) / per;
+    for (int64_t c = (int64_t)blockIdx.x * kSincWaves + wave; c < n_chunks; c += (int64_t)gridDim.x * kSincWaves) {
+        const int64_t l = c * per + lane;
+        // the weight is read first: a zero-weight line (a rejected resonance)
+        // costs nothing else, and the live ones are packed to the front
+        const float wl = (lane < per && l < n_lines) ? w[l] : 0.0f;
+        const uint64_t live = __ballot(wl != 0.0f);
+        const int n_live = __popcll(live);
+        if (n_live == 0) continue;
+        __builtin_amdgcn_wave_barrier();
         if (wl != 0.0f) {
-            const double al = a[l] * inv_pi;
-            s_ud[t] = make_double2(al * (E0 - E_r[l]), al * dE);
-        } else {
-            s_ud[t] = make_double2(0.0, 0.0);
+            SincLine o;
+            const double al = fabs(a[l]) * inv_pi, er = E_r[l];
+            o.u0 = al * (E0 - er);
+            o.du = al * dE;
+            sincospi(o.du - 2.0 * rint(0.5 * o.du), &o.sd, &o.cd);
+            const double inv_du = rcp_nr(o.du);
+            o.q = sqrt_nr((double)wl) * inv_pi * inv_du;
+            const double n = rint((er - E0) * inv_dE), u = fma(n, o.du, o.u0);
+            o.nf = (float)(n - (double)bin0);
+            o.f = (float)(u * inv_du);
+            o.w = wl;
+            // At the centre sine and distance vanish together.  The sine there is
+            // off by up to 1e-13 of the largest of the run, min(1, 8 pi du), and by
+            // the rounding of its phase, 1e-15 du: below 3e-8 of itself unless
+            // |u(n)| is under this line, where every cell is taken on its own
+            // (1 line in 1e4 at most).  So are negative weights and steps too
+            // small to divide by.
+            const double small = 4.0e-6 * fmin(1.0, 25.0 * fabs(o.du)) + 4.0e-8 * fabs(o.du);
+            o.direct = !(fabs(o.du) >= 1.0e-250) || wl < 0.0f || !(fabs(u) >= small);
+            lines[__popcll(live & ((1ULL << lane) - 1ULL))] = o;
         }
-        __syncthreads();
-        for (int q0 = 0; q0 < kLineTile; q0 += kSincGroup) {
-            const float4 w4 = s_w4[q0 / kSincGroup];
-            // uniform across the block: every thread reads the same slots
-            if (w4.x == 0.0f && w4.y == 0.0f && w4.z == 0.0f && w4.w == 0.0f) continue;
-            const float wg[kSincGroup] = {w4.x, w4.y, w4.z, w4.w};
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        for (int j0 = 0; j0 < n_live; j0 += kSincGroup) {
             float g[BINS];
 #pragma unroll
             for (int m = 0; m < BINS; ++m) g[m] = 0.0f;
+            const int j1 = j0 + kSincGroup < n_live ? j0 + kSincGroup : n_live;
+#pragma unroll 2
+            for (int j = j0; j < j1; ++j) {
+                const SincLine &o = lines[j];
+                if (__builtin_amdgcn_readfirstlane(o.direct)) {
+                    double k = kb - kMid;
+                    asm volatile("" : "+v"(k));  // keeps the run's bins out of registers outside this rare branch
 #pragma unroll
-            for (int j = 0; j < kSincGroup; ++j) {
-                const float wq = wg[j];
-                if (wq == 0.0f) continue;
-                const double2 ud = s_ud[q0 + j];
+                    for (int m = 0; m < BINS; ++m) {
+                        const double u = fma(k + m, o.du, o.u0);
+                        g[m] = fmaf(o.w, sinc2_cell((float)(u - rint(u)), (float)u), g[m]);
+                    }
+                    continue;
+                }
+                const double cd = o.cd, c2 = 2.0 * cd, q = o.q;
+                const double u = fma(kb, o.du, o.u0), r = u - rint(u), z = r * r;
+                const double S = (q * r) * horner(sin_r, z), C = q * horner(cos_r, z);
+                const float base = run0f - o.nf, f = o.f;
+                double up = S, lo = fma(S, cd, -C * o.sd);  // sines at the middle and one bin before
+                double up_p = lo, lo_p = up;
 #pragma unroll
-                for (int m = 0; m < BINS; ++m) {
-                    const double u = fma(kd[m], ud.y, ud.x);
-                    const float r = (float)(u - rint(u));
-                    g[m] = fmaf(wq, sinc2_cell(r, (float)u), g[m]);
+                for (int i = 0; i < kMid; ++i) {
+                    const int mu = kMid + i, ml = kMid - 1 - i;
+                    const float xu = (float)up * __builtin_amdgcn_rcpf((base + (float)mu) + f);
+                    const float xl = (float)lo * __builtin_amdgcn_rcpf((base + (float)ml) + f);
+                    g[mu] = fmaf(xu, xu, g[mu]);
+                    g[ml] = fmaf(xl, xl, g[ml]);
+                    const double un = fma(c2, up, -up_p), ln = fma(c2, lo, -lo_p);
+                    up_p = up;
+                    up = un;
+                    lo_p = lo;
+                    lo = ln;
                 }
             }
 #pragma unroll
             for (int m = 0; m < BINS; ++m) acc[m] += (double)g[m];
         }
+    }
+    // the block's partial row: its waves added in order
+    for (int v = 0; v < kSincWaves; ++v) {
+        if (wave == v) {
+#pragma unroll
+            for (int m = 0; m < BINS; ++m) s_sum[run0 + m] = v == 0 ? acc[m] : s_sum[run0 + m] + acc[m];
+        }
         __syncthreads();
     }
     double *out = partial + (int64_t)blockIdx.x * n_E;
-#pragma unroll
-    for (int m = 0; m < BINS; ++m) {
-        const int64_t k = bin0 + t + (int64_t)m * kRedThreads;
-        if (k < n_E) out[k] = acc[m];
-    }
+    for (int k = threadIdx.x; k < kWindow && bin0 + k < n_E; k += kSincBlock) out[bin0 + k] = s_sum[k];
 }
 
-// General grid: x = a (E_k - E_r) formed in FP64 per cell.
+// General grid: x = a (E_k - E_r) formed in FP64 per cell (E_grid null: the
+// degenerate uniform grid E0 + k dE whose step is zero or not finite).
 template <int BINS>
 __global__ void __launch_bounds__(kRedThreads) sincsq_general_kernel(
     const double *__restrict__ E_r, const double *__restrict__ a, const float *__restrict__ w,
-    int64_t n_lines, const double *__restrict__ E_grid, int64_t n_E, double *__restrict__ partial) {
+    int64_t n_lines, const double *__restrict__ E_grid, double E0, double dE, int64_t n_E,
+    double *__restrict__ partial) {
     __shared__ double s_er[kLineTile];
     __shared__ double s_a[kLineTile];
     __shared__ float s_w[kLineTile];
@@ -195,7 +285,7 @@ __global__ void __launch_bounds__(kRedThreads) sincsq_general_kernel(
     for (int m = 0; m < BINS; ++m) {
         acc[m] = 0.0;
         const int64_t k = bin0 + t + (int64_t)m * kRedThreads;
-        Ek[m] = k < n_E ? E_grid[k] : 0.0;
+        Ek[m] = k < n_E ? (E_grid ? E_grid[k] : E0 + (double)k * dE) : 0.0;
     }
     const double inv_pi = 1.0 / kPi;
     const int64_t n_tiles = (n_lines + kLineTile - 1) / kLineTile;
@@ -630,6 +720,61 @@ hr_status dense_plan(int64_t n_items, int64_t tile, int64_t n_E, DensePlan &P) {
     return HR_OK;
 }
 
+// Launch shape of the uniform-grid reduction.  The window of 64 `bins` bins is
+// the smallest cover of the grid in windows of 256 to 1024 bins, a window's
+// fixed cost per line counted as three bins per lane (the sine and cosine at the
+// middle of each run).  Four blocks of four waves share a CU; a wave takes chunks
+// of `per` lines, 64 where that leaves every resident wave four, fewer on small
+// inputs so that all of them work.  Dead lines come in runs, so where chunks
+// abound four times the resident blocks are launched to even the waves out
+// (2.7e6 lines on 1024 bins: 448 us resident, 402 so; 1.8e5 lines lose 20 us).
+struct SincPlan {
+    int bins = 16, per = kSincChunk;
+    int64_t gx = 1, windows = 1;
+    size_t bytes = 0;
+};
+hr_status sinc_plan(int64_t n_lines, int64_t n_E, SincPlan &P) {
+    int cu = 0;
+    hr_status st = device_cu(cu);
+    if (st != HR_OK) return st;
+    int64_t best = INT64_MAX;
+    for (int b = 16; b >= 4; b -= 4) {
+        const int64_t win = (n_E + 64 * b - 1) / (64 * b), cost = win * (b + 3);
+        if (cost < best) {
+            best = cost;
+            P.bins = b;
+            P.windows = win;
+        }
+    }
+    int64_t room = 4 * (int64_t)cu / (P.windows > 0 ? P.windows : 1);
+    room = room < 1 ? 1 : room;
+    while (P.per > 8 && n_lines < room * kSincWaves * P.per * 4) P.per /= 2;
+    if (P.per == kSincChunk) room *= 4;
+    const int64_t chunks = (n_lines + P.per - 1) / P.per;
+    const int64_t want = (chunks + kSincWaves - 1) / kSincWaves;
+    P.gx = want < room ? (want > 0 ? want : 1) : room;
+    P.bytes = (n_lines == 0 || n_E == 0) ? 0 : partial_bytes(P.gx, n_E);
+    return HR_OK;
+}
+
+// Whether the recurrence runs: a uniform grid with a step (every other grid
+// takes the general reducer).
+bool sinc_recurs(const hr_sincsq_args &p) { return p.uniform && p.dE != 0.0 && isfinite(p.dE) && isfinite(p.E0); }
+
+// Workspace bytes of hr_sincsq_reduce.
+hr_status sinc_bytes(const hr_sincsq_args &p, size_t &bytes) {
+    if (sinc_recurs(p)) {
+        SincPlan P;
+        hr_status st = sinc_plan(p.n_lines, p.n_E, P);
+        bytes = P.bytes;
+        return st;
+    }
+    DensePlan P;
+    hr_status st = dense_plan(p.n_lines, kLineTile, p.n_E, P);
+    bytes = P.bytes;
+    return st;
+}
+
 // Blocks of the standalone windowed reduction and its workspace bytes:
 // [partials blocks*4*n | spec n | node moments 9n].
 int64_t window_reduce_blocks(int cu, int64_t n_lines) {
@@ -681,24 +826,37 @@ extern "C" hr_status hr_sincsq_reduce(const hr_sincsq_args *args, void *stream) 
     if (p.n_lines == 0 || p.n_E == 0) return HR_OK;
     HR_REQUIRE(p.E_r && p.a && p.w && p.out, "hr_sincsq_reduce: null pointer");
     HR_REQUIRE(p.uniform || p.E_grid, "hr_sincsq_reduce: a non-uniform grid needs E_grid");
-    constexpr int BINS = kDenseBins;
+    hipStream_t s = (hipStream_t)stream;
+    void *ws = p.ws.ptr;
+    if (sinc_recurs(p)) {
+        SincPlan P;
+        hr_status st = sinc_plan(p.n_lines, p.n_E, P);
+        if (st != HR_OK) return st;
+        HR_REQUIRE_WS(p.ws, P.bytes, "hr_sincsq_reduce");
+        HR_REQUIRE(P.windows <= 65535, "hr_sincsq_reduce: %lld bins exceed one launch", (long long)p.n_E);
+        const dim3 grid((unsigned)P.gx, (unsigned)P.windows), block(kSincBlock);
+#define HR_SINC(B)                                                                                              \
+    hipLaunchKernelGGL(sincsq_uniform_kernel<B>, grid, block, 0, s, p.E_r, p.a, p.w, p.n_lines, P.per, p.E0,   \
+                       p.dE, p.n_E, (double *)ws)
+        switch (P.bins) {
+        case 4: HR_SINC(4); break;
+        case 8: HR_SINC(8); break;
+        case 12: HR_SINC(12); break;
+        default: HR_SINC(16); break;
+        }
+#undef HR_SINC
+        HR_CHECK_HIP(hipGetLastError());
+        return row_sum((const double *)ws, P.gx, p.n_E, p.out, s);
+    }
     DensePlan P;
     hr_status st = dense_plan(p.n_lines, kLineTile, p.n_E, P);
     if (st != HR_OK) return st;
     HR_REQUIRE_WS(p.ws, P.bytes, "hr_sincsq_reduce");
-    const int64_t gx = P.gx;
-    void *ws = p.ws.ptr;
-    hipStream_t s = (hipStream_t)stream;
-    dim3 grid((unsigned)gx, (unsigned)P.bin_tiles);
-    if (p.uniform) {
-        hipLaunchKernelGGL(sincsq_uniform_kernel<BINS>, grid, dim3(kRedThreads), 0, s, p.E_r, p.a, p.w,
-                           p.n_lines, p.E0, p.dE, p.n_E, (double *)ws);
-    } else {
-        hipLaunchKernelGGL(sincsq_general_kernel<BINS>, grid, dim3(kRedThreads), 0, s, p.E_r, p.a, p.w,
-                           p.n_lines, p.E_grid, p.n_E, (double *)ws);
-    }
+    const dim3 grid((unsigned)P.gx, (unsigned)P.bin_tiles);
+    hipLaunchKernelGGL(sincsq_general_kernel<kDenseBins>, grid, dim3(kRedThreads), 0, s, p.E_r, p.a, p.w, p.n_lines,
+                       p.uniform ? nullptr : p.E_grid, p.E0, p.dE, p.n_E, (double *)ws);
     HR_CHECK_HIP(hipGetLastError());
-    return row_sum((const double *)ws, gx, p.n_E, p.out, s);
+    return row_sum((const double *)ws, P.gx, p.n_E, p.out, s);
 }
 
 // Scratch of hr_sincsq_reduce_static: the partial spectra of one call live in
@@ -735,11 +893,14 @@ extern "C" hr_status hr_sincsq_reduce_static(const hr_sincsq_args *args, void *s
     HR_REQUIRE(args != nullptr, "hr_sincsq_reduce_static: null args");
     HR_REQUIRE(args->n_lines >= 0 && args->n_E >= 0, "hr_sincsq_reduce_static: negative size");
     if (args->n_lines == 0 || args->n_E == 0) return HR_OK;
+    // the sizes taken are those whose general-grid partials (and 64 more rows) fit, whatever the grid
     DensePlan P;
+    size_t need = 0;
     hr_status st = dense_plan(args->n_lines, kLineTile, args->n_E, P);
+    if (st == HR_OK) st = sinc_bytes(*args, need);
     if (st != HR_OK) return st;
-    // the sizes taken are those whose partials and 64 rows more fit
-    const size_t need = partial_bytes(P.gx + (P.gx < 64 ? P.gx : 64), args->n_E);
+    const size_t limit = partial_bytes(P.gx + (P.gx < 64 ? P.gx : 64), args->n_E);
+    if (need < limit) need = limit;
     HR_REQUIRE(need <= (size_t)HR_SINCSQ_STATIC_SCRATCH_BYTES,
                "hr_sincsq_reduce_static: %lld bins need %zu bytes of partials, more than the %zu-byte static "
                "scratch (use hr_sincsq_reduce with a workspace)",
@@ -757,11 +918,7 @@ extern "C" hr_status hr_sincsq_workspace_bytes(const hr_sincsq_args *args, size_
     using namespace hr;
     HR_REQUIRE(args != nullptr && bytes != nullptr, "hr_sincsq_workspace_bytes: null argument");
     HR_REQUIRE(args->n_lines >= 0 && args->n_E >= 0, "hr_sincsq_workspace_bytes: negative size");
-    DensePlan P;
-    hr_status st = dense_plan(args->n_lines, kLineTile, args->n_E, P);
-    if (st != HR_OK) return st;
-    *bytes = P.bytes;
-    return HR_OK;
+    return sinc_bytes(*args, *bytes);
 }
 
 extern "C" hr_status hr_brem_workspace_bytes(const hr_brem_args *args, size_t *bytes) {

@@ -206,7 +206,7 @@ struct PoissonTerm {
     __device__ __forceinline__ void init(double mean, double draw) {
         lam = mean;
         u = mean > 0.0 ? draw : -1.0;  // no draw, no events
-        p = exp_neg(mean);
+        p = exp_any(-mean);
         cdf = p;
         n = 0;
     }

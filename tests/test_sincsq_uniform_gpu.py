@@ -1,0 +1,80 @@
+"""The uniform-grid sinc^2 reduction at the edges of its windows, runs and chunks (GPU).
+
+Against the FP64 profile in numpy.  The bound: a cell's factor x carries the
+rounding of the sine, the two of the distance, the reciprocal's ulp and the
+product (6 x 2^-24), squared and summed in FP32 groups of four, 1e-6 of the sum
+in all; the stepped sines are off by at most 1e-10 of their envelope, which a
+square turns into 2e-10 of the envelope (w at the centre, w/(pi u)^2 beyond)."""
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _lines(rng, n, E0, dE, n_E):
+    """Lines across the grid and beyond it, of every width: far narrower than a bin
+    to far wider than the grid; some centred on a bin or half way, some without
+    weight, one flat (a = 0) and one of negative weight."""
+    E_r = E0 + dE * rng.uniform(-1.5 * n_E - 3, 2.5 * n_E + 3, n)
+    on = rng.random(n)
+    k = rng.integers(0, n_E, n)
+    E_r = np.where(on < 0.2, E0 + dE * k, np.where(on < 0.3, E0 + dE * (k + 0.5), E_r))
+    a = np.exp(rng.uniform(np.log(1e-9), np.log(2e3), n)) / abs(dE)
+    w = np.where(rng.random(n) < 0.2, 0.0, rng.uniform(1e-3, 1.0, n)).astype(np.float32)
+    if n > 6:
+        a[3] = 0.0
+        w[3], w[5] = 0.5, -0.25
+    return E_r, a, w
+
+
+def _reduce(E_r, a, w, E0, dE, n_E, device):
+    import torch
+
+    from pyrite_amd import _lib
+
+    t = [torch.as_tensor(v, device=device) for v in (E_r, a, w)]
+    out = torch.full((n_E,), 0.125, dtype=torch.float64, device=device)
+    args = _lib.SincsqArgs()
+    args.n_lines, args.E_r, args.a, args.w = E_r.size, *(v.data_ptr() for v in t)
+    args.n_E, args.E_grid, args.uniform, args.E0, args.dE = n_E, None, 1, E0, dE
+    args.out = out.data_ptr()
+    args.ws = _lib.DeviceScratch(device).get(_lib.workspace_bytes("hr_sincsq_workspace_bytes", C.byref(args)))
+    _lib.check(_lib.load().hr_sincsq_reduce(C.byref(args), C.c_void_p(torch.cuda.current_stream().cuda_stream)),
+               "hr_sincsq_reduce")
+    return out.cpu().numpy() - 0.125
+
+
+@pytest.mark.parametrize("n_E", [1, 2, 63, 64, 255, 256, 257, 777, 1024, 1025, 1400, 3001])
+@pytest.mark.parametrize("n_lines", [1, 8, 9, 700, 40_000])
+def test_uniform_reduction_matches_fp64(device, n_E, n_lines):
+    rng = np.random.default_rng([n_E, n_lines])
+    E0, dE = 1000.0, (47.9, -3.5)[n_E % 2]
+    if n_lines > 1000 and n_E > 1100:
+        n_lines = 5000
+    E_r, a, w = _lines(rng, n_lines, E0, dE, n_E)
+    got = _reduce(E_r, a, w, E0, dE, n_E, device)
+    k = np.arange(n_E)
+    want, envelope = np.zeros(n_E), np.zeros(n_E)
+    for s in range(0, n_lines, 4096):
+        al = (a[s:s + 4096] / np.pi)[:, None]
+        u = k[None, :] * (al * dE) + al * (E0 - E_r[s:s + 4096])[:, None]
+        wl = w[s:s + 4096].astype(float)[:, None]
+        r = u - np.rint(u)
+        cell = np.where(u == 0.0, 1.0, np.sin(np.pi * r) / (np.pi * np.where(u == 0.0, 1.0, u))) ** 2
+        want += (wl * cell).sum(0)
+        envelope += (np.abs(wl) / np.maximum(1.0, (np.pi * u) ** 2)).sum(0)
+        want_abs = (np.abs(wl) * cell).sum(0) if s == 0 else want_abs + (np.abs(wl) * cell).sum(0)
+    assert np.isfinite(got).all()
+    assert np.all(np.abs(got - want) <= 1e-6 * want_abs + 1e-9 * envelope + 1e-15), \
+        float(np.max(np.abs(got - want) / (1e-6 * want_abs + 1e-9 * envelope + 1e-15)))
+
+
+def test_step_of_zero_takes_the_general_reducer(device):
+    """A uniform grid whose bins coincide: every bin the same profile."""
+    E_r, a, w = np.array([10.0, 12.0]), np.array([0.7, 0.2]), np.array([1.0, 0.5], dtype=np.float32)
+    got = _reduce(E_r, a, w, 11.0, 0.0, 5, device)
+    want = float((w * np.sinc(a * (11.0 - E_r) / np.pi) ** 2).sum())
+    np.testing.assert_allclose(got, want, rtol=1e-6)
