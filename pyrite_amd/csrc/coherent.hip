@@ -79,27 +79,29 @@ __global__ void __launch_bounds__(256) coherent_lines_kernel(hr_coherent_args a,
 #pragma unroll
             for (int f = 0; f < kRecFields; ++f) r[f] = 0.0;
             if (o.keep) {
-                const double amp = sqrt(kAlpha * o.omega / (4.0 * kPi * kPi * kHbarc));
+                constexpr double kPref = kAlpha / (4.0 * kPi * kPi * kHbarc);
+                const double amp = sqrt(kPref * o.omega);
                 // formation_coefficients(L_start mu, L_end mu)
                 const double tau0 = k.path0 * o.mu, tau1 = k.path1 * o.mu;
                 const double q = 0.25 * (tau1 - tau0);
                 double apb, bma;
                 if (fabs(q) < kFormationSmallQ) {
-                    const double c0 = exp(-0.25 * (tau0 + tau1));
+                    const double c0 = exp_any(-0.25 * (tau0 + tau1));
                     apb = 2.0 * c0 * cosh(q);
                     bma = -2.0 * c0 * sinh(q);
                 } else {
-                    const double ea = exp(-0.5 * tau0), eb = exp(-0.5 * tau1);
+                    const double ea = exp_any(-0.5 * tau0), eb = exp_any(-0.5 * tau1);
                     apb = ea + eb;
                     bma = eb - ea;
                 }
                 // _recoil_formation_line: exact vacuum centre, width, recoil phase shifts
                 const double numerator = o.vdg - o.r_num;
                 const double denom = k.denom_row + o.r_den;
-                const double E_c = kHbarc * numerator / denom;
-                const double x = numerator / denom * k.inv_E;
-                const double kappa = 1.0 / (1.0 - x);
-                const double a_vac = kappa * denom * k.t_L / (2.0 * kHbarc);
+                const double ratio = numerator * rcp_nr(denom);
+                const double E_c = kHbarc * ratio;
+                const double x = ratio * k.inv_E;
+                const double kappa = rcp_nr(1.0 - x);
+                const double a_vac = kappa * denom * k.t_L * (1.0 / (2.0 * kHbarc));
                 const double d_shift = kappa * (x * k.denom_row + o.r_den) * age;
                 const double g_shift = kappa * (x * o.vdg - o.r_num) * age;
                 const double Gx = p.g[3 * g], Gy = p.g[3 * g + 1], Gz = p.g[3 * g + 2];
@@ -112,7 +114,7 @@ __global__ void __launch_bounds__(256) coherent_lines_kernel(hr_coherent_args a,
                 if (good) {
                     r[0] = E_c;
                     r[1] = a_vac;
-                    r[2] = (d_geom + d_shift) / kHbarc;
+                    r[2] = (d_geom + d_shift) * (1.0 / kHbarc);
                     r[3] = rx * Gx + ry * Gy + rz * Gz + g_shift;
                     r[4] = cs_re;
                     r[5] = cs_im;

@@ -52,11 +52,12 @@ __device__ __forceinline__ void segment_lines(const hr_line_args &p, int64_t j, 
             for (int pol = 0; pol < 2; ++pol) A2 += o.A_re[pol] * o.A_re[pol] + o.A_im[pol] * o.A_im[pol];
             // _batched.py:702-728 + _fused.py:267-281, one piece, fraction 1
             const double T_abs = mean_transmission(k.path0 * o.mu, k.path1 * o.mu);
-            const double pref = kAlpha * o.omega / (4.0 * kPi * kPi * kHbarc) * (k.t_L * k.t_L) * T_abs;
+            constexpr double kPref = kAlpha / (4.0 * kPi * kPi * kHbarc);
+            const double pref = kPref * o.omega * (k.t_L * k.t_L) * T_abs;
             const double wt = pref * A2 * p.wm[g];
             if (isfinite(wt) && wt > 0.0) {
                 w = wt * dir_w;
-                a_width = o.slope * k.t_L / (2.0 * kHbarc);
+                a_width = o.slope * k.t_L * (1.0 / (2.0 * kHbarc));
                 Er = o.E_res;
             }
         }
@@ -514,7 +515,7 @@ struct WindowShared {
 static_assert(sizeof(WindowShared) <= 160 * 1024, "window LDS");
 
 __device__ __forceinline__ double tail_value(double m2, double m3, double m4, double x) {
-    const double inv = 1.0 / x;
+    const double inv = rcp_nr(x);
     return (m2 + (m3 + m4 * inv) * inv) * inv * inv;
 }
 
@@ -525,15 +526,17 @@ __device__ __forceinline__ double sincsq_cell(double u) {
 
 struct WindowGrid {
     int64_t n;
-    double E0, dE, x_c;
+    double E0, dE, x_c, inv_dE;
 };
 
 __device__ __forceinline__ void window_line(WindowShared &sh, double *__restrict__ dep_far, const WindowGrid &G,
                                             double Er, double a, double w) {
     const int64_t n = G.n;
-    const double nd = rint((Er - G.E0) / G.dE);
+    // quotients rounded as divisions: they decide the line's node and reach
+    const double inv_a = rcp_nr(a);
+    const double nd = rint(div_by(Er - G.E0, G.dE, G.inv_dE));
     const double eps = Er - (G.E0 + nd * G.dE);
-    double R = ceil((fabs(eps) + G.x_c / a) / G.dE);
+    double R = ceil(div_by(fabs(eps) + div_by(G.x_c, a, inv_a), G.dE, G.inv_dE));
     R = fmin(R, 4503599627370496.0);
     const int64_t node = (int64_t)nd;
     const bool conv_range = node + n >= 0 && node + n < 3 * n;
@@ -549,7 +552,7 @@ __device__ __forceinline__ void window_line(WindowShared &sh, double *__restrict
             conv = true;
         }
     }
-    const double m2 = 0.5 / (a * a);
+    const double m2 = 0.5 * inv_a * inv_a;
     const double m3 = 2.0 * eps * m2, m4 = 3.0 * eps * eps * m2;
     const double inv_pi = 1.0 / kPi;
     const double al = a * inv_pi;
@@ -973,6 +976,7 @@ hr_status window_setup(int64_t n_E, double E0, double dE, double x_c, WindowGrid
     G.E0 = E0;
     G.dE = dE;
     G.x_c = x_c;
+    G.inv_dE = 1.0 / dE;
     return HR_OK;
 }
 
