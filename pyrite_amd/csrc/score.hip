@@ -508,9 +508,14 @@ __global__ void __launch_bounds__(kRedThreads) brem_kernel(hr_brem_args p, doubl
 constexpr int kWinThreads = HR_WINDOW_THREADS;
 constexpr int kWinMaxBins = 4096;
 
+struct WindowItem {
+    double Er, a, w;
+};
+
 struct WindowShared {
     double spec[kWinMaxBins];
     double dep[3][kWinMaxBins];
+    WindowItem queue[kWinThreads / 64][64];  // each wave's lines of longer windows
 };
 static_assert(sizeof(WindowShared) <= 160 * 1024, "window LDS");
 
@@ -529,50 +534,113 @@ struct WindowGrid {
     double E0, dE, x_c, inv_dE;
 };
 
-__device__ __forceinline__ void window_line(WindowShared &sh, double *__restrict__ dep_far, const WindowGrid &G,
-                                            double Er, double a, double w) {
+// Where a line deposits: bins [lo, hi] exactly, the tail moments at its node
+// where `conv` (a window of less than a quarter of the grid, node in reach).
+struct WindowPlan {
+    double Er, al, m2, m3, m4;  // al = a/pi
+    int64_t node, lo, hi;
+    bool conv;
+};
+
+__device__ __forceinline__ WindowPlan window_plan(const WindowGrid &G, double Er, double a) {
     const int64_t n = G.n;
+    WindowPlan P;
+    P.Er = Er;
+    P.al = a * (1.0 / kPi);
     // quotients rounded as divisions: they decide the line's node and reach
     const double inv_a = rcp_nr(a);
     const double nd = rint(div_by(Er - G.E0, G.dE, G.inv_dE));
     const double eps = Er - (G.E0 + nd * G.dE);
     double R = ceil(div_by(fabs(eps) + div_by(G.x_c, a, inv_a), G.dE, G.inv_dE));
     R = fmin(R, 4503599627370496.0);
-    const int64_t node = (int64_t)nd;
-    const bool conv_range = node + n >= 0 && node + n < 3 * n;
-    int64_t lo = 0, hi = n - 1;
-    bool conv = false;
-    if (conv_range) {
+    P.node = (int64_t)nd;
+    P.lo = 0;
+    P.hi = n - 1;
+    P.conv = false;
+    if (P.node + n >= 0 && P.node + n < 3 * n) {
         const int64_t RR = (int64_t)R;
-        const int64_t l = node - RR < 0 ? 0 : node - RR;
-        const int64_t h = node + RR > n - 1 ? n - 1 : node + RR;
+        const int64_t l = P.node - RR < 0 ? 0 : P.node - RR;
+        const int64_t h = P.node + RR > n - 1 ? n - 1 : P.node + RR;
         if ((double)(h - l + 1) < 0.25 * (double)n) {
-            lo = l;
-            hi = h;
-            conv = true;
+            P.lo = l;
+            P.hi = h;
+            P.conv = true;
         }
     }
-    const double m2 = 0.5 * inv_a * inv_a;
-    const double m3 = 2.0 * eps * m2, m4 = 3.0 * eps * eps * m2;
-    const double inv_pi = 1.0 / kPi;
-    const double al = a * inv_pi;
-    for (int64_t e = lo; e <= hi; ++e) {
-        double v = sincsq_cell(al * ((G.E0 + (double)e * G.dE) - Er));
-        if (conv && e != node) v -= tail_value(m2, m3, m4, (double)(e - node) * G.dE);
+    P.m2 = 0.5 * inv_a * inv_a;
+    P.m3 = 2.0 * eps * P.m2;
+    P.m4 = 3.0 * eps * eps * P.m2;
+    return P;
+}
+
+// Bins lo + first, lo + first + step, ... of a line's window.
+__device__ __forceinline__ void window_cells(WindowShared &sh, const WindowGrid &G, const WindowPlan &P, double w,
+                                             int first, int step) {
+    for (int64_t e = P.lo + first; e <= P.hi; e += step) {
+        double v = sincsq_cell(P.al * ((G.E0 + (double)e * G.dE) - P.Er));
+        if (P.conv && e != P.node) v -= tail_value(P.m2, P.m3, P.m4, (double)(e - P.node) * G.dE);
         atomicAdd(&sh.spec[e], w * v);
     }
-    if (conv) {
-        if (node >= 0 && node < n) {
-            atomicAdd(&sh.dep[0][node], w * m2);
-            atomicAdd(&sh.dep[1][node], w * m3);
-            atomicAdd(&sh.dep[2][node], w * m4);
-        } else {
-            const int64_t L = 3 * n;
-            atomicAdd(&dep_far[node + n], w * m2);
-            atomicAdd(&dep_far[L + node + n], w * m3);
-            atomicAdd(&dep_far[2 * L + node + n], w * m4);
-        }
+}
+
+__device__ __forceinline__ void window_moments(WindowShared &sh, double *__restrict__ dep_far, const WindowGrid &G,
+                                               const WindowPlan &P, double w) {
+    const int64_t n = G.n, node = P.node;
+    if (node >= 0 && node < n) {
+        atomicAdd(&sh.dep[0][node], w * P.m2);
+        atomicAdd(&sh.dep[1][node], w * P.m3);
+        atomicAdd(&sh.dep[2][node], w * P.m4);
+    } else {
+        const int64_t L = 3 * n;
+        atomicAdd(&dep_far[node + n], w * P.m2);
+        atomicAdd(&dep_far[L + node + n], w * P.m3);
+        atomicAdd(&dep_far[2 * L + node + n], w * P.m4);
     }
+}
+
+// Deposits one line per lane (w == 0: none); every lane of the wave takes part.
+// A window's length goes as 1/L: most lines cover a few bins, one in hundreds the
+// whole grid, and a lane that walked its own held the other 63 up (12,007
+// segments x 64 reflections x 64 rays: 5.6 to 35 ms by the draw of lengths, 2.2
+// to 2.4 so).  Windows of up to kOwnCells bins stay with their lane; longer ones
+// go through the wave's queue, four at a time to 16 lanes each, and those above
+// kGroupCells to the whole wave.
+constexpr int kOwnCells = 8, kGroupCells = 128, kGroupLanes = 16;
+
+__device__ __forceinline__ void window_deposit(WindowShared &sh, double *__restrict__ dep_far,
+                                               const WindowGrid &G, double Er, double a, float wf) {
+    const int lane = __lane_id();
+    WindowItem *queue = sh.queue[threadIdx.x >> 6];
+    const double w = (double)wf;
+    const bool live = wf != 0.0f && a > 0.0;
+    int64_t cells = 0;
+    if (live) {
+        const WindowPlan P = window_plan(G, Er, a);
+        cells = P.hi - P.lo + 1;
+        if (P.conv) window_moments(sh, dep_far, G, P, w);
+        if (cells <= kOwnCells) window_cells(sh, G, P, w, 0, 1);
+    }
+    const uint64_t queued = __ballot(cells > kOwnCells);
+    if (queued == 0) return;
+    uint64_t wide = __ballot(cells > kGroupCells);
+    const int n = __popcll(queued);
+    __builtin_amdgcn_wave_barrier();
+    if (cells > kOwnCells) queue[__popcll(queued & ((1ULL << lane) - 1ULL))] = WindowItem{Er, a, w};
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    for (int i = lane / kGroupLanes; i < n; i += 64 / kGroupLanes) {
+        const WindowItem it = queue[i];
+        const WindowPlan P = window_plan(G, it.Er, it.a);
+        if (P.hi - P.lo + 1 <= kGroupCells) window_cells(sh, G, P, it.w, lane % kGroupLanes, kGroupLanes);
+    }
+    while (wide != 0) {
+        const int l = __ffsll((unsigned long long)wide) - 1;
+        wide &= wide - 1;
+        const WindowItem it = queue[__popcll(queued & ((1ULL << l) - 1ULL))];
+        window_cells(sh, G, window_plan(G, it.Er, it.a), it.w, lane, 64);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
 __device__ __forceinline__ void window_zero(WindowShared &sh, int64_t n) {
@@ -606,11 +674,12 @@ __global__ void __launch_bounds__(kWinThreads) window_lines_kernel(hr_line_args 
     const int64_t j0 = (int64_t)blockIdx.x * per;
     const int64_t j1 = j0 + per < p.n_seg ? j0 + per : p.n_seg;
     double *far = dep_far + (int64_t)d * 9 * G.n;
-    for (int64_t j = j0 + threadIdx.x; j < j1; j += blockDim.x) {
-        segment_lines(p, j, d, [&](int, double Er, double a_width, double w64) {
-            const float wf = (float)w64;  // the line weight the dense route stores
-            if (wf == 0.0f || !(a_width > 0.0)) return;
-            window_line(sh, far, G, Er, a_width, (double)wf);
+    // whole waves: the lanes past the end carry the last segment without weight
+    for (int64_t jw = j0 + (threadIdx.x & ~63); jw < j1; jw += blockDim.x) {
+        const int64_t j = jw + (threadIdx.x & 63);
+        segment_lines(p, j < j1 ? j : j1 - 1, d, [&](int, double Er, double a_width, double w64) {
+            // the line weight the dense route stores
+            window_deposit(sh, far, G, Er, a_width, j < j1 ? (float)w64 : 0.0f);
         });
     }
     __syncthreads();
@@ -626,11 +695,11 @@ __global__ void __launch_bounds__(kWinThreads) window_given_kernel(const double 
     __shared__ WindowShared sh;
     window_zero(sh, G.n);
     __syncthreads();
-    for (int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; l < n_lines;
-         l += (int64_t)gridDim.x * blockDim.x) {
-        const float wf = w[l];
-        if (wf == 0.0f || !(a[l] > 0.0)) continue;
-        window_line(sh, dep_far, G, E_r[l], a[l], (double)wf);
+    for (int64_t lw = (int64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63); lw < n_lines;
+         lw += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t l = lw + (threadIdx.x & 63);
+        const float wf = l < n_lines ? w[l] : 0.0f;
+        window_deposit(sh, dep_far, G, wf != 0.0f ? E_r[l] : 0.0, wf != 0.0f ? a[l] : 0.0, wf);
     }
     __syncthreads();
     window_flush(sh, G.n, partial + (int64_t)blockIdx.x * 4 * G.n);
