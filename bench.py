@@ -295,7 +295,8 @@ def coherent_case(args):
                    "histories_per_step": cfg.Ne, "segments_per_history": pipe.segments / max(pipe.histories, 1),
                    "grouped_term": bool(args.coherent_grouped)},
         "roofline": {
-            "kernel": "hr_coherent_field: coherent_field_kernel + field_partials_kernel",
+            "kernel": "hr_coherent_both: coherent_grouped_kernel + row_sum_kernel" if cfg.coherent_grouped
+                      else "hr_coherent_field: coherent_field_kernel + row_sum_kernel",
             "bound": "valu", "pipe": "vector ALU, FP32 peak (FP64 phase reduction counted as FP32 work)",
             "achieved": achieved, "peak": roofline.PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
             "frac": achieved / roofline.PEAK_FP32_TFLOPS, "traffic": None,

@@ -650,6 +650,11 @@ typedef struct hr_coherent_grouped_args {
 } hr_coherent_grouped_args;
 hr_status hr_coherent_grouped(const hr_coherent_grouped_args *args, void *stream);
 hr_status hr_coherent_grouped_workspace_bytes(const hr_coherent_grouped_args *args, size_t *bytes);
+/* hr_coherent_grouped and hr_coherent_field of the same lines in one pass: the
+ * lines of the groups (all of them where the groups cover [0, n_lines)) are also
+ * added to field.field.  Its own workspace size. */
+hr_status hr_coherent_both(const hr_coherent_grouped_args *args, void *stream);
+hr_status hr_coherent_both_workspace_bytes(const hr_coherent_grouped_args *args, size_t *bytes);
 /* out[k] += scale sum_d dir_weight[d] sum_g wm[g] M_dg(k), with P = |F_s|^2 + |F_p|^2
  * of the all-line field, G the grouped term and F = factor[k]:
  * pair_scale < 0 (sampled bunch): M = (1 - F) G + F P;

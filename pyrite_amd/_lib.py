@@ -469,6 +469,8 @@ SIGNATURES = {
     "hr_coherent_finalize": (C.c_int32, [_dp, C.c_int32, C.c_int32, _dp, _dp, C.c_int64, C.c_double, _dp, _dp]),
     "hr_coherent_grouped": (C.c_int32, [C.POINTER(CoherentGroupedArgs), _dp]),
     "hr_coherent_grouped_workspace_bytes": (C.c_int32, [C.POINTER(CoherentGroupedArgs), C.POINTER(C.c_size_t)]),
+    "hr_coherent_both": (C.c_int32, [C.POINTER(CoherentGroupedArgs), _dp]),
+    "hr_coherent_both_workspace_bytes": (C.c_int32, [C.POINTER(CoherentGroupedArgs), C.POINTER(C.c_size_t)]),
     "hr_coherent_blend_finalize": (C.c_int32, [_dp, _dp, C.c_int32, C.c_int32, _dp, _dp, C.c_int64, _dp, C.c_double,
                                                C.c_double, _dp, _dp]),
     "hr_vr_round": (C.c_int32, [C.POINTER(TransportArgs), C.c_int32, _dp, _dp]),

@@ -222,11 +222,11 @@ __device__ __forceinline__ void field_cell(const FieldTile &T, int l, const doub
     }
 }
 
-// acc += the fields of tile lines [0, nt), in FP32 groups of kFieldGroup lines.
+// acc += the fields of tile lines [first, nt), in FP32 groups of kFieldGroup lines.
 template <int BINS>
-__device__ __forceinline__ void tile_fields(const FieldTile &T, int nt, const double (&E)[BINS],
+__device__ __forceinline__ void tile_fields(const FieldTile &T, int first, int nt, const double (&E)[BINS],
                                             const double (&D)[BINS], double (&acc)[BINS][4]) {
-    for (int l0 = 0; l0 < nt; l0 += kFieldGroup) {
+    for (int l0 = first; l0 < nt; l0 += kFieldGroup) {
         float g[BINS][4];
 #pragma unroll
         for (int m = 0; m < BINS; ++m)
@@ -279,7 +279,7 @@ __global__ void __launch_bounds__(kFieldThreads) coherent_field_kernel(hr_cohere
         __syncthreads();
         if (tid < nt) stage_line(T, R, plane, j0 + tid, tid);
         __syncthreads();
-        tile_fields<BINS>(T, nt, E, D, acc);
+        tile_fields<BINS>(T, 0, nt, E, D, acc);
     }
 #pragma unroll
     for (int m = 0; m < BINS; ++m) {
@@ -296,12 +296,18 @@ __global__ void __launch_bounds__(kFieldThreads) coherent_field_kernel(hr_cohere
 // Block (chunk s, row r, bin window w): groups [n_groups s / S, n_groups (s+1) / S)
 // of row r, each group's columns [gs[e], gs[e+1]) summed to one FP64 field
 // whose |F_s|^2 + |F_p|^2 is added to the thread's bins; writes its partial
-// (or adds it when S == 1).
-template <int BINS>
+// (or adds it when S == 1).  Lines are staged kFieldTile at a time whatever the
+// groups (a history holds some twenty), and a group closes where its columns end.
+// With kField the groups' fields are added up too, the flat field of the same
+// lines: one evaluation of each cell serves both (81,000 lines x 4 rows x 1,024
+// bins: 340 us flat and 404 us grouped as two launches; the call from rows to
+// blended spectrum 845 us so, 526 us with one).
+template <int BINS, bool kField>
 __global__ void __launch_bounds__(kFieldThreads) coherent_grouped_kernel(hr_coherent_field_args p,
                                                                          const int64_t *__restrict__ gs,
                                                                          int64_t n_groups, int W, int S,
-                                                                         double *__restrict__ out) {
+                                                                         double *__restrict__ out,
+                                                                         double *__restrict__ field) {
     __shared__ FieldTile T;
     const int tid = threadIdx.x;
     const int row = (int)(blockIdx.y / W), win = (int)(blockIdx.y % W);
@@ -316,31 +322,47 @@ __global__ void __launch_bounds__(kFieldThreads) coherent_grouped_kernel(hr_cohe
         E[m] = valid[m] ? p.E_grid[k] : 0.0;
         D[m] = valid[m] ? p.dom[k] : 0.0;
     }
-    double G[BINS];
+    double G[BINS], acc[BINS][4], flat[BINS][4];
 #pragma unroll
-    for (int m = 0; m < BINS; ++m) G[m] = 0.0;
+    for (int m = 0; m < BINS; ++m) {
+        G[m] = 0.0;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[m][c] = flat[m][c] = 0.0;
+    }
     const int64_t plane = (int64_t)p.n_rows * p.ld;
     const double *R = p.rec + (int64_t)row * p.ld;
     const int64_t g_lo = n_groups * split / S, g_hi = n_groups * (split + 1) / S;
-    for (int64_t grp = g_lo; grp < g_hi; ++grp) {
-        int64_t b = gs[grp], e = gs[grp + 1];
-        b = b < 0 ? 0 : (b > p.n_lines ? p.n_lines : b);
-        e = e < b ? b : (e > p.n_lines ? p.n_lines : e);
-        double acc[BINS][4];
+    auto column = [&](int64_t g) {
+        const int64_t c = gs[g];
+        return c < 0 ? 0 : (c > p.n_lines ? p.n_lines : c);
+    };
+    int64_t grp = g_lo, closes = column(grp + 1 <= n_groups ? grp + 1 : n_groups);
+    const int64_t end = column(g_hi);
+    for (int64_t t0 = column(g_lo); t0 < end; t0 += kFieldTile) {
+        const int nt = (int)(end - t0 < kFieldTile ? end - t0 : kFieldTile);
+        __syncthreads();
+        if (tid < nt) stage_line(T, R, plane, t0 + tid, tid);
+        __syncthreads();
+        for (int l = 0; l < nt;) {
+            int stop = nt;
+            if (closes - t0 < nt) stop = closes - t0 > l ? (int)(closes - t0) : l;
+            tile_fields<BINS>(T, l, stop, E, D, acc);
+            l = stop;
+            while (grp < g_hi && closes <= t0 + l) {
 #pragma unroll
-        for (int m = 0; m < BINS; ++m)
+                for (int m = 0; m < BINS; ++m) {
+                    G[m] += acc[m][0] * acc[m][0] + acc[m][1] * acc[m][1] + acc[m][2] * acc[m][2] +
+                            acc[m][3] * acc[m][3];
 #pragma unroll
-            for (int c = 0; c < 4; ++c) acc[m][c] = 0.0;
-        for (int64_t j0 = b; j0 < e; j0 += kFieldTile) {
-            const int nt = (int)(e - j0 < kFieldTile ? e - j0 : kFieldTile);
-            __syncthreads();
-            if (tid < nt) stage_line(T, R, plane, j0 + tid, tid);
-            __syncthreads();
-            tile_fields<BINS>(T, nt, E, D, acc);
+                    for (int c = 0; c < 4; ++c) {
+                        if (kField) flat[m][c] += acc[m][c];
+                        acc[m][c] = 0.0;
+                    }
+                }
+                ++grp;
+                closes = grp < g_hi ? column(grp + 1) : INT64_MAX;
+            }
         }
-#pragma unroll
-        for (int m = 0; m < BINS; ++m)
-            G[m] += acc[m][0] * acc[m][0] + acc[m][1] * acc[m][1] + acc[m][2] * acc[m][2] + acc[m][3] * acc[m][3];
     }
 #pragma unroll
     for (int m = 0; m < BINS; ++m) {
@@ -348,6 +370,13 @@ __global__ void __launch_bounds__(kFieldThreads) coherent_grouped_kernel(hr_cohe
         const int64_t k = ((int64_t)win * BINS + m) * kFieldThreads + tid;
         if (S == 1) out[(int64_t)row * n_E + k] += G[m];
         else out[((int64_t)split * p.n_rows + row) * n_E + k] = G[m];
+        if constexpr (kField) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                if (S == 1) field[((int64_t)row * 4 + c) * n_E + k] += flat[m][c];
+                else field[(((int64_t)split * p.n_rows + row) * 4 + c) * n_E + k] = flat[m][c];
+            }
+        }
     }
 }
 
@@ -428,14 +457,15 @@ hr_status field_plan(const hr_coherent_field_args &p, FieldPlan &P) {
 }
 
 // Launch shape of hr_coherent_grouped: S chunks of groups (as the field plan,
-// never more than there are groups), partials of n_rows*n_E cells.
-hr_status grouped_plan(const hr_coherent_field_args &p, int64_t n_groups, FieldPlan &P) {
+// never more than there are groups), partials of n_rows*n_E cells, and four
+// times as many more with the flat field.
+hr_status grouped_plan(const hr_coherent_field_args &p, int64_t n_groups, bool field, FieldPlan &P) {
     int cu = 0;
     hr_status st = device_cu(cu);
     if (st != HR_OK) return st;
     const int64_t per_block = (int64_t)kFieldThreads * kFieldBins;
     P.W = (p.n_E + per_block - 1) / per_block;
-    const int64_t cells = (int64_t)p.n_rows * p.n_E;
+    const int64_t cells = (int64_t)p.n_rows * p.n_E * (field ? 5 : 1);
     int64_t S = (int64_t)cu * 8 / ((int64_t)p.n_rows * P.W);
     if (S > n_groups) S = n_groups;
     const int64_t s_cap = (int64_t)(kMaxPartialBytes / ((size_t)cells * sizeof(double)));
@@ -443,6 +473,53 @@ hr_status grouped_plan(const hr_coherent_field_args &p, int64_t n_groups, FieldP
     if (S < 1) S = 1;
     P.S = S;
     P.bytes = (S > 1 && n_groups > 0) ? (size_t)S * (size_t)cells * sizeof(double) : 0;
+    return HR_OK;
+}
+
+// hr_coherent_grouped, with the flat field of the same lines added to
+// args->field.field where `field` is set.
+hr_status grouped_run(const hr_coherent_grouped_args *args, bool field, const char *who, void *stream) {
+    HR_REQUIRE(args != nullptr, "%s: null args", who);
+    const hr_coherent_field_args &p = args->field;
+    const int64_t n_groups = args->n_groups;
+    HR_REQUIRE(p.n_lines >= 0 && p.ld >= p.n_lines && p.n_rows >= 1 && p.n_E >= 1 && n_groups >= 0,
+               "%s: bad sizes (n_lines=%lld ld=%lld n_rows=%d n_E=%lld n_groups=%lld)", who, (long long)p.n_lines,
+               (long long)p.ld, p.n_rows, (long long)p.n_E, (long long)n_groups);
+    if (p.n_lines == 0 || n_groups == 0) return HR_OK;
+    HR_REQUIRE(p.rec && p.E_grid && p.dom && args->group_start && args->grouped && (!field || p.field),
+               "%s: null pointer", who);
+    FieldPlan P;
+    hr_status st = grouped_plan(p, n_groups, field, P);
+    if (st != HR_OK) return st;
+    const int64_t W = P.W, S = P.S;
+    const int64_t cells = (int64_t)p.n_rows * p.n_E;
+    HR_REQUIRE((int64_t)p.n_rows * W <= 65535, "%s: %lld row windows exceed the grid", who,
+               (long long)(p.n_rows * W));
+    HR_REQUIRE_WS(p.ws, P.bytes, who);
+    hipStream_t s = (hipStream_t)stream;
+    double *ws = (double *)p.ws.ptr;
+    double *out = S > 1 ? ws : args->grouped, *flat = S > 1 ? ws + S * cells : p.field;
+    const dim3 grid((unsigned)S, (unsigned)(p.n_rows * W));
+    if (field)
+        hipLaunchKernelGGL((coherent_grouped_kernel<kFieldBins, true>), grid, dim3(kFieldThreads), 0, s, p,
+                           args->group_start, n_groups, (int)W, (int)S, out, flat);
+    else
+        hipLaunchKernelGGL((coherent_grouped_kernel<kFieldBins, false>), grid, dim3(kFieldThreads), 0, s, p,
+                           args->group_start, n_groups, (int)W, (int)S, out, nullptr);
+    HR_CHECK_HIP(hipGetLastError());
+    if (S == 1) return HR_OK;
+    st = row_sum(out, S, cells, args->grouped, s);
+    return st != HR_OK || !field ? st : row_sum(flat, S, 4 * cells, p.field, s);
+}
+
+hr_status grouped_bytes(const hr_coherent_grouped_args *args, bool field, const char *who, size_t *bytes) {
+    HR_REQUIRE(args != nullptr && bytes != nullptr, "%s: null argument", who);
+    const hr_coherent_field_args &p = args->field;
+    HR_REQUIRE(p.n_lines >= 0 && p.n_rows >= 1 && p.n_E >= 1 && args->n_groups >= 0, "%s: bad sizes", who);
+    FieldPlan P;
+    hr_status st = grouped_plan(p, args->n_groups, field, P);
+    if (st != HR_OK) return st;
+    *bytes = P.bytes;
     return HR_OK;
 }
 
@@ -534,44 +611,21 @@ extern "C" hr_status hr_coherent_finalize(const double *field, int32_t n_dir, in
 }
 
 extern "C" hr_status hr_coherent_grouped_workspace_bytes(const hr_coherent_grouped_args *args, size_t *bytes) {
-    using namespace hr;
-    HR_REQUIRE(args != nullptr && bytes != nullptr, "hr_coherent_grouped_workspace_bytes: null argument");
-    const hr_coherent_field_args &p = args->field;
-    HR_REQUIRE(p.n_lines >= 0 && p.n_rows >= 1 && p.n_E >= 1 && args->n_groups >= 0,
-               "hr_coherent_grouped_workspace_bytes: bad sizes");
-    FieldPlan P;
-    hr_status st = grouped_plan(p, args->n_groups, P);
-    if (st != HR_OK) return st;
-    *bytes = P.bytes;
-    return HR_OK;
+    return hr::grouped_bytes(args, false, "hr_coherent_grouped_workspace_bytes", bytes);
 }
 
 extern "C" hr_status hr_coherent_grouped(const hr_coherent_grouped_args *args, void *stream) {
     HR_TRACE("hr_coherent_grouped");
-    using namespace hr;
-    HR_REQUIRE(args != nullptr, "hr_coherent_grouped: null args");
-    const hr_coherent_field_args &p = args->field;
-    const int64_t n_groups = args->n_groups;
-    HR_REQUIRE(p.n_lines >= 0 && p.ld >= p.n_lines && p.n_rows >= 1 && p.n_E >= 1 && n_groups >= 0,
-               "hr_coherent_grouped: bad sizes (n_lines=%lld ld=%lld n_rows=%d n_E=%lld n_groups=%lld)",
-               (long long)p.n_lines, (long long)p.ld, p.n_rows, (long long)p.n_E, (long long)n_groups);
-    if (p.n_lines == 0 || n_groups == 0) return HR_OK;
-    HR_REQUIRE(p.rec && p.E_grid && p.dom && args->group_start && args->grouped,
-               "hr_coherent_grouped: null pointer");
-    FieldPlan P;
-    hr_status st = grouped_plan(p, n_groups, P);
-    if (st != HR_OK) return st;
-    const int64_t W = P.W, S = P.S;
-    const int64_t cells = (int64_t)p.n_rows * p.n_E;
-    HR_REQUIRE((int64_t)p.n_rows * W <= 65535, "hr_coherent_grouped: %lld row windows exceed the grid",
-               (long long)(p.n_rows * W));
-    HR_REQUIRE_WS(p.ws, P.bytes, "hr_coherent_grouped");
-    hipStream_t s = (hipStream_t)stream;
-    double *out = S > 1 ? (double *)p.ws.ptr : args->grouped;
-    hipLaunchKernelGGL(coherent_grouped_kernel<kFieldBins>, dim3((unsigned)S, (unsigned)(p.n_rows * W)),
-                       dim3(kFieldThreads), 0, s, p, args->group_start, n_groups, (int)W, (int)S, out);
-    HR_CHECK_HIP(hipGetLastError());
-    return S > 1 ? row_sum((const double *)p.ws.ptr, S, cells, args->grouped, s) : HR_OK;
+    return hr::grouped_run(args, false, "hr_coherent_grouped", stream);
+}
+
+extern "C" hr_status hr_coherent_both_workspace_bytes(const hr_coherent_grouped_args *args, size_t *bytes) {
+    return hr::grouped_bytes(args, true, "hr_coherent_both_workspace_bytes", bytes);
+}
+
+extern "C" hr_status hr_coherent_both(const hr_coherent_grouped_args *args, void *stream) {
+    HR_TRACE("hr_coherent_both");
+    return hr::grouped_run(args, true, "hr_coherent_both", stream);
 }
 
 extern "C" hr_status hr_coherent_blend_finalize(const double *field, const double *grouped, int32_t n_dir,

@@ -165,32 +165,47 @@ class CoherentScorer:
         a.rec = rec.data_ptr()
         _lib.check(self.lib.hr_coherent_lines(C.byref(a), _stream()), "hr_coherent_lines")
 
-    def _launch_field(self, rec, n_lines):
-        f = _lib.CoherentFieldArgs()
+    def _field_args(self, f, rec, n_lines):
         f.rec, f.ld, f.n_lines, f.n_rows = rec.data_ptr(), int(n_lines), int(n_lines), self.n_rows
         f.n_E, f.E_grid, f.dom = self.n_E, self.lines.E_grid_d.data_ptr(), self.dom.data_ptr()
         f.field = self.field.data_ptr()
-        f.ws = self.scratch.get(_lib.workspace_bytes("hr_coherent_field_workspace_bytes", C.byref(f)))
-        ev = None
-        if self.record_events:
-            import torch
 
-            ev = (torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True))
-            ev[0].record()
-        _lib.check(self.lib.hr_coherent_field(C.byref(f), _stream()), "hr_coherent_field")
-        if ev is not None:
-            ev[1].record()
-            self.events.append((ev, n_lines * self.n_rows * self.n_E))
+    def _timed(self, launch, n_lines):
+        """``launch()``, between events when recording."""
+        if not self.record_events:
+            return launch()
+        import torch
+
+        ev = (torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True))
+        ev[0].record()
+        launch()
+        ev[1].record()
+        self.events.append((ev, n_lines * self.n_rows * self.n_E))
+
+    def _launch_field(self, rec, n_lines):
+        f = _lib.CoherentFieldArgs()
+        self._field_args(f, rec, n_lines)
+        f.ws = self.scratch.get(_lib.workspace_bytes("hr_coherent_field_workspace_bytes", C.byref(f)))
+        self._timed(lambda: _lib.check(self.lib.hr_coherent_field(C.byref(f), _stream()), "hr_coherent_field"),
+                    n_lines)
 
     def _launch_grouped(self, rec, n_lines, group_start):
+        """The grouped term alone."""
         g = _lib.CoherentGroupedArgs()
-        f = g.field
-        f.rec, f.ld, f.n_lines, f.n_rows = rec.data_ptr(), int(n_lines), int(n_lines), self.n_rows
-        f.n_E, f.E_grid, f.dom = self.n_E, self.lines.E_grid_d.data_ptr(), self.dom.data_ptr()
+        self._field_args(g.field, rec, n_lines)
         g.group_start, g.n_groups = group_start.data_ptr(), int(group_start.numel()) - 1
         g.grouped = self.grouped.data_ptr()
-        f.ws = self.scratch.get(_lib.workspace_bytes("hr_coherent_grouped_workspace_bytes", C.byref(g)))
+        g.field.ws = self.scratch.get(_lib.workspace_bytes("hr_coherent_grouped_workspace_bytes", C.byref(g)))
         _lib.check(self.lib.hr_coherent_grouped(C.byref(g), _stream()), "hr_coherent_grouped")
+
+    def _launch_both(self, rec, n_lines, group_start):
+        """The flat field and the grouped term of the same lines."""
+        g = _lib.CoherentGroupedArgs()
+        self._field_args(g.field, rec, n_lines)
+        g.group_start, g.n_groups = group_start.data_ptr(), int(group_start.numel()) - 1
+        g.grouped = self.grouped.data_ptr()
+        g.field.ws = self.scratch.get(_lib.workspace_bytes("hr_coherent_both_workspace_bytes", C.byref(g)))
+        self._timed(lambda: _lib.check(self.lib.hr_coherent_both(C.byref(g), _stream()), "hr_coherent_both"), n_lines)
 
     def add_rows(self, rows, seg_count, n, slots, live_counts=None, electron=None):
         """Add the fields of ``n`` particles' slot rows (``slots`` rows each,
@@ -232,18 +247,18 @@ class CoherentScorer:
                 off = incl[i0:i1] - cnt[i0:i1] - base
                 rec = self._records(n_lines)
                 self._launch_lines(rows, seg_count, off, i0, i1 - i0, slots, rec, n_lines)
-                if live_counts is None:
+                if live_counts is None and self.grouped is None:
                     self._launch_field(rec, n_lines)
-                    if self.grouped is not None:
-                        if key is None:
-                            starts = off
-                        else:
-                            k = key[i0:i1]
-                            first = np.flatnonzero(np.r_[True, k[1:] != k[:-1]])
-                            starts = off[torch.as_tensor(first, device=off.device)]
-                        group_start = torch.cat((starts.to(torch.int64),
-                                                 torch.tensor([n_lines], dtype=torch.int64, device=off.device)))
-                        self._launch_grouped(rec, n_lines, group_start)
+                elif live_counts is None:
+                    if key is None:
+                        starts = off
+                    else:
+                        k = key[i0:i1]
+                        first = np.flatnonzero(np.r_[True, k[1:] != k[:-1]])
+                        starts = off[torch.as_tensor(first, device=off.device)]
+                    group_start = torch.cat((starts.to(torch.int64),
+                                             torch.tensor([n_lines], dtype=torch.int64, device=off.device)))
+                    self._launch_both(rec, n_lines, group_start)
                 else:
                     coeff = rec[: N_FIELDS * self.n_rows * n_lines].view(N_FIELDS, self.n_rows, n_lines)[4:8]
                     live_counts.append(int((coeff != 0).any(0).sum().item()))
