@@ -340,24 +340,282 @@ constexpr float kLn2f = 0.69314718055994531f;
 constexpr double kLn2d = 0.6931471805599453;
 
 // BH+Elwert brem over segment tiles (brem.py:396-423, brem_jit_kernel.py:76-153).
-constexpr int kBremTile = 128;
+//
+// A cell is A g(T, k) e(path, mu_k): the segment's length and weight, the Born
+// cross section with its Elwert factors, which depend on the energy and the bin
+// alone, and the mean escape.  The kernel is bound by vector instructions, 40 a
+// cell.  g is smooth in T away from the spectral tip, so rows of one energy class,
+// an eighth of an octave, can take it as a polynomial of degree 6 per bin, through
+// seven Chebyshev points of the class evaluated in FP64: 23 instructions a cell.
+// The nearest singularity is T = k: a class c +- h with (c - k) >= 8 h interpolates
+// to 16^-7 = 4e-9 of g; closer classes (energies below about twice the bin's)
+// evaluate every cell.
+//
+// So the rows are first ordered by class, those that add nothing dropped (a stable
+// counting sort: the order, and with it the sum, is fixed), and the polynomials of
+// the classes that occur are laid out, 30 us in three launches, from kBremSortCells
+// cells on.  Before (one order, four tiles of 128 rows to a block) and now, us:
+// 150,000 rows of 0.5..5 MeV x 1,024 bins 234 -> 143 (222 unordered), 150,001 of
+// 5 keV..10 MeV x 2,000 with a quarter dead 271 -> 230 (268), 1e6 of 5 keV..5 MeV x
+// 1,024 990 -> 720 (976); below the limit 60,000 x 1,024 93 -> 79 (82 ordered),
+// 150,000 x 300 125 -> 87 (103), 20,000 x 1,024 92 -> 48.
+constexpr int kBremStage = 128;  // rows staged at a time
+constexpr int kBremDeg = 6, kBremNodes = kBremDeg + 1;
+constexpr double kBremReach = 8.0;
+constexpr int64_t kBremSortCells = 100'000'000;
+
+// Chebyshev points x_i = cos(pi (2i + 1)/14) of [-1, 1] and, row j, the weights of
+// the values there in coefficient j of the polynomial through them.
+__constant__ const double kNode[kBremNodes] = {0.97492791218182361, 0.78183148246802981, 0.43388373911755812, 0.0,
+                                               -0.43388373911755812, -0.78183148246802981, -0.97492791218182361};
+__constant__ const double kNodeWeight[kBremNodes][kBremNodes] = {
+    {0.0, 0.0, 0.0, 1.0, 0.0, 0.0, 0.0},
+    {0.22824347439014988, -0.79747338888240381, 2.0765213965723364, 0.0, -2.0765213965723364, 0.79747338888240381,
+     -0.22824347439014988},
+    {0.23411318061389407, -1.0200067492357776, 4.7858935686218833, -8.0, 4.7858935686218833, -1.0200067492357776,
+     0.23411318061389407},
+    {-1.5858139578511551, 5.0751495106189253, -5.5818117994536827, 0.0, 5.5818117994536827, -5.0751495106189253,
+     1.5858139578511551},
+    {-1.6265961185809208, 6.4913598702856729, -12.864763751704752, 16.0, -12.864763751704752, 6.4913598702856729,
+     -1.6265961185809208},
+    {1.9834685216802656, -4.4568133128311934, 3.5740867769967075, 0.0, -3.5740867769967075, 4.4568133128311934,
+     -1.9834685216802656},
+    {2.0344771104577316, -5.7004781884227062, 8.2374296493935458, -9.1428571428571423, 8.2374296493935458,
+     -5.7004781884227062, 2.0344771104577316}};
+
+// Energy class of a row: eight to an octave from 1/4 keV up (the exponent and top
+// three mantissa bits), the last for rows that add nothing.
+constexpr int kBremClasses = 128;
+constexpr uint32_t kBremClass0 = 0x3e800000u >> 20;
+
+// Centre and half width of a class, and whether its rows may take polynomials up
+// to photon energy k_hi (the first and last classes are open ended).
+struct BremBand {
+    double c, h;
+    __device__ __forceinline__ explicit BremBand(int cls) {
+        const double lo = __uint_as_float((kBremClass0 + cls) << 20), hi = __uint_as_float((kBremClass0 + cls + 1) << 20);
+        c = 0.5 * (lo + hi);
+        h = 0.5 * (hi - lo);
+    }
+    __device__ __forceinline__ static bool closed(int cls) { return cls > 0 && cls < kBremClasses - 2; }
+    __device__ __forceinline__ bool reaches(double k) const { return c - k >= kBremReach * h; }
+};
+
+__device__ __forceinline__ int brem_class(float T, float L, float w) {
+    if ((double)w * (double)L == 0.0) return kBremClasses - 1;
+    const int c = (int)(__float_as_uint(fmaxf(T, 0.25f)) >> 20) - (int)kBremClass0;
+    return c < 0 ? 0 : (c > kBremClasses - 2 ? kBremClasses - 2 : c);
+}
+
+// The wave's class counts (kScatter false), or its rows written where `at` says
+// the next row of each class goes: rows [b per, (b + 1) per) of wave b.
+template <bool kScatter>
+__device__ __forceinline__ void brem_order(const hr_brem_args &p, int64_t per, int64_t b, uint32_t *s_at,
+                                           uint32_t *__restrict__ order) {
+    const int lane = threadIdx.x;
+    const int64_t end = (b + 1) * per < p.n_seg ? (b + 1) * per : p.n_seg;
+    for (int64_t j0 = b * per; j0 < end; j0 += 64) {
+        const int64_t j = j0 + lane;
+        const bool in = j < end;
+        const int c = in ? brem_class(p.E_keV[j], p.L[j], p.row_weight ? p.row_weight[j] : 1.0f) : 0;
+        uint64_t same = __ballot(in);  // the lanes of this lane's class
+#pragma unroll
+        for (int bit = 0; bit < 7; ++bit) {
+            const uint64_t set = __ballot((c >> bit) & 1);
+            same &= ((c >> bit) & 1) ? set : ~set;
+        }
+        const uint32_t rank = (uint32_t)__popcll(same & ((1ULL << lane) - 1ULL));
+        const uint32_t at = in ? s_at[c] : 0u;
+        __syncthreads();
+        if (in && kScatter) order[at + rank] = (uint32_t)j;
+        if (in && rank == 0) s_at[c] = at + (uint32_t)__popcll(same);
+        __syncthreads();
+    }
+}
+
+// counts[class][wave]
+__global__ void __launch_bounds__(64) brem_count_kernel(hr_brem_args p, int64_t per, uint32_t *__restrict__ counts) {
+    __shared__ uint32_t s_at[kBremClasses];
+    for (int c = threadIdx.x; c < kBremClasses; c += 64) s_at[c] = 0u;
+    __syncthreads();
+    brem_order<false>(p, per, blockIdx.x, s_at, nullptr);
+    for (int c = threadIdx.x; c < kBremClasses; c += 64) counts[c * (int64_t)gridDim.x + blockIdx.x] = s_at[c];
+}
+
+// Exclusive sums over the waves of each class, and the classes' totals.  One wave per class.
+__global__ void __launch_bounds__(64) brem_scan_kernel(uint32_t *__restrict__ counts, int64_t waves,
+                                                       uint32_t *__restrict__ totals) {
+    uint32_t *C = counts + blockIdx.x * waves;
+    const int lane = threadIdx.x;
+    uint32_t sum = 0;
+    for (int64_t i0 = 0; i0 < waves; i0 += 64) {
+        const uint32_t v = i0 + lane < waves ? C[i0 + lane] : 0u;
+        uint32_t incl = v;
+#pragma unroll
+        for (int d = 1; d < 64; d *= 2) {
+            const uint32_t up = __shfl_up(incl, d);
+            incl += lane >= d ? up : 0u;
+        }
+        if (i0 + lane < waves) C[i0 + lane] = sum + incl - v;
+        sum += __shfl(incl, 63);
+    }
+    if (lane == 0) totals[blockIdx.x] = sum;
+}
+
+// Exclusive sums of f(total) over the classes, by one wave; the whole sum in [kBremClasses].
+template <class F>
+__device__ __forceinline__ void brem_class_sums(const uint32_t *__restrict__ totals, uint32_t *out, F f) {
+    const int lane = __lane_id();
+    const uint32_t a = f(totals[2 * lane]), b = f(totals[2 * lane + 1]);
+    uint32_t incl = a + b;
+#pragma unroll
+    for (int d = 1; d < 64; d *= 2) {
+        const uint32_t up = __shfl_up(incl, d);
+        incl += lane >= d ? up : 0u;
+    }
+    out[2 * lane] = incl - a - b;
+    out[2 * lane + 1] = incl - b;
+    if (lane == 63) out[kBremClasses] = incl;
+}
+
+// The first `waves` blocks write the rows in class order; the others, eight bins of
+// one class each, lay out the polynomials of g in the place of T within its class,
+// poly[class][power][bin], for the classes that occur and the bins they reach: one
+// lane per node and bin.
+constexpr int kBremPolyBins = 8;
+__global__ void __launch_bounds__(64) brem_lay_kernel(hr_brem_args p, int64_t per, int64_t waves,
+                                                      const uint32_t *__restrict__ counts,
+                                                      const uint32_t *__restrict__ totals,
+                                                      uint32_t *__restrict__ order, float *__restrict__ poly) {
+    __shared__ uint32_t s_at[kBremClasses + 1];
+    const int lane = threadIdx.x;
+    if (blockIdx.x < waves) {
+        brem_class_sums(totals, s_at, [](uint32_t n) { return n; });
+        __syncthreads();
+        for (int c = lane; c < kBremClasses; c += 64) s_at[c] += counts[c * waves + blockIdx.x];
+        __syncthreads();
+        brem_order<true>(p, per, blockIdx.x, s_at, order);
+        return;
+    }
+    const int64_t groups = (p.n_E + kBremPolyBins - 1) / kBremPolyBins, at = blockIdx.x - waves;
+    const int cls = (int)(at / groups);
+    const int node = lane / kBremPolyBins;
+    const int64_t k = at % groups * kBremPolyBins + lane % kBremPolyBins;
+    if (!BremBand::closed(cls) || totals[cls] == 0) return;
+    const BremBand band(cls);
+    const double kev = k < p.n_E ? p.E_grid_eV[k] * 1.0e-3 : 0.0;
+    double v = 0.0;
+    if (kev > 0.0 && band.reaches(kev) && node < kBremNodes) {
+        const double T = band.c + band.h * kNode[node], Tf = T - kev, Tm = Tf + 2.0 * kMc2;
+        const double pi_ = sqrt_nr(T * (T + 2.0 * kMc2)) * (1.0 / kMc2);
+        const double inv_bi = (1.0 + T * (1.0 / kMc2)) * rcp_nr(pi_);
+        const double TT = Tf * Tm, rs = rsqrt_nr(TT), spf = pi_ + TT * rs * (1.0 / kMc2);
+        const double rcp_bf = rs * (kMc2 + Tf);
+        const double born = ln(spf * spf * (kMc2 * kMc2) * rcp_nr(kev * (T + Tm)));
+        double sum = 0.0;
+        for (int el = 0; el < p.n_el; ++el) {
+            // n (16/3) alpha r_e^2 Z^2 beta_i (1 - exp(-2 pi Z alpha/beta_i)) / (1 - exp(-2 pi Z alpha/beta_f))
+            const double z = 2.0 * kPi * kAlpha * p.Z[el];
+            sum += p.n_cm3[el] * p.Z[el] * p.Z[el] * (1.0 - exp_any(-z * inv_bi)) * rcp_nr(1.0 - exp_any(-z * rcp_bf));
+        }
+        const double front = (16.0 / 3.0) * kAlpha * kReCm2 * rcp_nr(pi_ * pi_ * inv_bi * (kev * 1.0e3));
+        v = front * born * rcp_bf * sum;
+    }
+    double coef = 0.0;
+#pragma unroll
+    for (int i = 0; i < kBremNodes; ++i)
+        coef += kNodeWeight[node < kBremNodes ? node : 0][i] * __shfl(v, i * kBremPolyBins + lane % kBremPolyBins);
+    if (k < p.n_E && node < kBremNodes) poly[((int64_t)cls * kBremNodes + node) * p.n_E + k] = (float)coef;
+}
+
+// The rows of a tile: `rows` rows of one class where the rows are in class order,
+// of all rows as they lie where not.
+struct BremOrder {
+    const uint32_t *order, *totals;  // rows in class order; rows of each class
+    const float *poly;
+};
+
+struct BremTile {
+    int64_t r0, r1;
+    int cls;    // -1 without the order
+    bool band;  // rows that take the polynomials in this window of bins
+};
+
+struct BremShared {
+    uint32_t tile[kBremClasses + 1], first[kBremClasses + 1];  // of each class: first tile, first row
+    float k_max[kRedThreads / 64];
+};
+
+// Tile blockIdx.x of the window whose bins end at k_hi [keV] (this thread's bins;
+// the block's are joined here).
+template <bool kOrdered>
+__device__ __forceinline__ BremTile brem_tile(const hr_brem_args &p, int64_t rows, const BremOrder &o, float k_hi,
+                                              BremShared &sh) {
+    const int t = threadIdx.x;
+    const int64_t tile = blockIdx.x;
+    if (!kOrdered) {
+        const int64_t r0 = tile * rows;
+        return {r0, r0 + rows < p.n_seg ? r0 + rows : p.n_seg, -1, false};
+    }
+    if (t < 64) brem_class_sums(o.totals, sh.first, [](uint32_t n) { return n; });
+    else if (t < 128)
+        brem_class_sums(o.totals, sh.tile, [rows](uint32_t n) { return (uint32_t)((n + rows - 1) / rows); });
+#pragma unroll
+    for (int d = 32; d > 0; d /= 2) k_hi = fmaxf(k_hi, __shfl_xor(k_hi, d));
+    if ((t & 63) == 0) sh.k_max[t >> 6] = k_hi;
+    __syncthreads();
+    k_hi = fmaxf(fmaxf(sh.k_max[0], sh.k_max[1]), fmaxf(sh.k_max[2], sh.k_max[3]));
+    if (tile >= (int64_t)sh.tile[kBremClasses - 1]) return {0, 0, -1, false};
+    int lo = 0, hi = kBremClasses - 2;  // the last class that starts by this tile holds it
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if ((int64_t)sh.tile[mid] <= tile) lo = mid;
+        else hi = mid - 1;
+    }
+    const int64_t r0 = (int64_t)sh.first[lo] + (tile - sh.tile[lo]) * rows, end = sh.first[lo + 1];
+    return {r0, r0 + rows < end ? r0 + rows : end, lo, BremBand::closed(lo) && BremBand(lo).reaches((double)k_hi)};
+}
+
+// Length of segment j with its weight, and the shorter and longer of its escape paths:
+// from its two ends along n_hat (segment_escape.py:190-211).
+struct BremRow {
+    double wL, plo, phi;
+    __device__ __forceinline__ BremRow(const hr_brem_args &p, int64_t j) {
+        const double L = (double)p.L[j], half = 0.5 * L;
+        wL = (p.row_weight ? (double)p.row_weight[j] : 1.0) * L;
+        const double rz = p.r_mid[3 * j + 2], vz = p.v_hat[3 * j + 2];
+        const double p0 = slab_path(rz - half * vz, p.thickness, p.n_hat[2]);
+        const double p1 = slab_path(rz + half * vz, p.thickness, p.n_hat[2]);
+        plo = fmin(p0, p1);
+        phi = fmax(p0, p1);
+    }
+};
+
+constexpr int kBremGroup = 8;  // cells summed in FP32 (positive terms: rounding below 5e-7) before each FP64 add
+
+// Tile blockIdx.x of window blockIdx.y, to its partial row; thread t owns bins
+// t + kRedThreads m of the window.
 // NEL: element count of the composition (1..4), a template parameter so the
 // per-element loop unrolls with its constants in registers.
-template <int BINS, int NEL>
-__global__ void __launch_bounds__(kRedThreads) brem_kernel(hr_brem_args p, double *__restrict__ partial) {
-    // per staged segment: kinetic energy, momentum, the shorter and longer
-    // escape paths from its two ends along n_hat, their mean and difference,
-    // the per-element prefactors and whether any of them is nonzero
-    __shared__ float s_T[kBremTile], s_pi[kBremTile], s_plo[kBremTile], s_phi[kBremTile], s_pmid[kBremTile],
-        s_dp[kBremTile];
-    __shared__ float s_pref[kBremTile * 4];
-    __shared__ int s_live[kBremTile];
+template <int BINS, int NEL, bool kOrdered>
+__global__ void __launch_bounds__(kRedThreads, kOrdered && NEL == 4 ? 3 : 4) brem_kernel(hr_brem_args p, int64_t rows, BremOrder o,
+                                                              double *__restrict__ partial) {
+    // per staged segment: kinetic energy (its place in the class), momentum (length
+    // times weight, 1e-8 L w), the shorter and longer escape paths, their mean and
+    // difference; of rows evaluated cell by cell also the per-element prefactors and
+    // whether any of them is nonzero
+    __shared__ float s_T[kBremStage], s_pi[kBremStage], s_plo[kBremStage], s_phi[kBremStage], s_pmid[kBremStage],
+        s_dp[kBremStage];
+    __shared__ float s_pref[kBremStage * 4];
+    __shared__ int s_live[kBremStage];
+    __shared__ BremShared sh;
     const int t = threadIdx.x;
     const int64_t bin0 = (int64_t)blockIdx.y * kRedThreads * BINS;
     constexpr int n_el = NEL;
     double acc[BINS];
     // per-bin constants: k [keV], k / m^2 [1/keV], ln 2 / k [1/eV], mu, mu log2(e)
     float keV[BINS], k_m2[BINS], ln2_inv_k[BINS], mu[BINS], mu2[BINS];
+    float k_hi = 0.0f;
 #pragma unroll
     for (int m = 0; m < BINS; ++m) {
         acc[m] = 0.0;
@@ -366,78 +624,96 @@ __global__ void __launch_bounds__(kRedThreads) brem_kernel(hr_brem_args p, doubl
         keV[m] = (float)(kev * 1.0e-3);
         k_m2[m] = (float)(kev * 1.0e-3 / (kMc2 * kMc2));
         ln2_inv_k[m] = (float)(kLn2d / fmax(kev, 1.0e-30));
-        mu[m] = k < p.n_E ? p.mu[k] : 0.0f;
+        mu[m] = kev > 0.0 ? p.mu[k] : 0.0f;  // no cell otherwise
         mu2[m] = (float)((double)mu[m] * kLog2e);
+        k_hi = fmaxf(k_hi, keV[m] * (1.0f + 1.0e-6f));
+    }
+    const BremTile tile = brem_tile<kOrdered>(p, rows, o, k_hi, sh);
+    float g[BINS][kBremNodes];
+    double c = 0.0, inv_h = 0.0;
+    if (kOrdered && tile.band) {
+        const BremBand band(tile.cls);
+        c = band.c;
+        inv_h = 1.0 / band.h;
+#pragma unroll
+        for (int m = 0; m < BINS; ++m) {
+            const int64_t k = bin0 + t + (int64_t)m * kRedThreads;
+#pragma unroll
+            for (int i = 0; i < kBremNodes; ++i)
+                g[m][i] = k < p.n_E ? o.poly[((int64_t)tile.cls * kBremNodes + i) * p.n_E + k] : 0.0f;
+        }
     }
     float zi2[4];
     for (int el = 0; el < 4; ++el)  // exp(-2 pi Z alpha / beta) = exp2(-(2 pi Z alpha log2 e) / beta)
         zi2[el] = el < n_el ? (float)(2.0 * kPi * p.Z[el] * kAlpha * kLog2e) : 0.0f;
-    const int64_t n_tiles = (p.n_seg + kBremTile - 1) / kBremTile;
-    for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-        if (t < kBremTile) {
-            const int64_t j = tile * kBremTile + t;
-            if (j < p.n_seg) {
-                const float T = p.E_keV[j];
+    for (int64_t s0 = tile.r0; s0 < tile.r1; s0 += kBremStage) {
+        const int cnt = (int)(tile.r1 - s0 < kBremStage ? tile.r1 - s0 : kBremStage);
+        __syncthreads();
+        if (t < cnt) {
+            const int64_t j = kOrdered ? (int64_t)o.order[s0 + t] : s0 + t;
+            const BremRow row(p, j);
+            const float T = p.E_keV[j];
+            s_plo[t] = (float)row.plo;
+            s_phi[t] = (float)row.phi;
+            s_pmid[t] = (float)(0.5 * (row.plo + row.phi));
+            s_dp[t] = (float)(row.phi - row.plo);
+            if (kOrdered && tile.band) {
+                s_T[t] = (float)(((double)T - c) * inv_h);
+                s_pi[t] = (float)(row.wL * 1.0e-8);
+            } else {
                 const float pi_ = sqrtf(T * (T + 2.0f * (float)kMc2)) / (float)kMc2;
                 const float bi = pi_ / (1.0f + T / (float)kMc2);
                 s_T[t] = T;
                 s_pi[t] = pi_;
-                // escape paths from both ends along n_hat (segment_escape.py:190-211)
-                const double half = 0.5 * (double)p.L[j];
-                const double rz = p.r_mid[3 * j + 2], vz = p.v_hat[3 * j + 2];
-                const double p0 = slab_path(rz - half * vz, p.thickness, p.n_hat[2]);
-                const double p1 = slab_path(rz + half * vz, p.thickness, p.n_hat[2]);
-                const double plo = fmin(p0, p1), phi = fmax(p0, p1);
-                s_plo[t] = (float)plo;
-                s_phi[t] = (float)phi;
-                s_pmid[t] = (float)(0.5 * (plo + phi));
-                s_dp[t] = (float)(phi - plo);
                 int live = 0;
-                for (int el = 0; el < 4; ++el) {
-                    float pref = 0.0f;
-                    if (el < n_el) {
-                        // n L 1e-8 (16/3) alpha r_e^2 Z^2 beta_i (1 - exp(-2 pi Z alpha/beta_i)) / p_i^2
-                        const double den_i = 1.0 - exp(-2.0 * kPi * p.Z[el] * kAlpha / (double)bi);
-                        const double rw = p.row_weight ? (double)p.row_weight[j] : 1.0;
-                        pref = (float)(rw * p.n_cm3[el] * (double)p.L[j] * 1.0e-8 * (16.0 / 3.0) * kAlpha * kReCm2 *
-                                       p.Z[el] * p.Z[el] * (double)bi * den_i / ((double)pi_ * (double)pi_));
-                    }
+                for (int el = 0; el < n_el; ++el) {
+                    // n L 1e-8 (16/3) alpha r_e^2 Z^2 beta_i (1 - exp(-2 pi Z alpha/beta_i)) / p_i^2
+                    const double den_i = 1.0 - exp(-2.0 * kPi * p.Z[el] * kAlpha / (double)bi);
+                    const float pref =
+                        (float)(row.wL * p.n_cm3[el] * 1.0e-8 * (16.0 / 3.0) * kAlpha * kReCm2 * p.Z[el] * p.Z[el] *
+                                (double)bi * den_i / ((double)pi_ * (double)pi_));
                     s_pref[t * 4 + el] = pref;
                     live |= pref != 0.0f;
                 }
                 s_live[t] = live;
-            } else {
-                s_T[t] = 0.0f;
-                s_pi[t] = 0.0f;
-                s_plo[t] = 0.0f;
-                s_phi[t] = 0.0f;
-                s_pmid[t] = 0.0f;
-                s_dp[t] = 0.0f;
-                for (int el = 0; el < 4; ++el) s_pref[t * 4 + el] = 0.0f;
-                s_live[t] = 0;
             }
         }
         __syncthreads();
-        const int64_t left = p.n_seg - tile * kBremTile;
-        const int cnt = left < kBremTile ? (int)left : kBremTile;
-        // cells of kGroup segments are summed in FP32 (8 positive terms: relative
-        // rounding below 5e-7) before each FP64 accumulate
-        constexpr int kGroup = 8;
         float part[BINS];
 #pragma unroll
         for (int m = 0; m < BINS; ++m) part[m] = 0.0f;
         for (int q = 0; q < cnt; ++q) {
-            if ((q & (kGroup - 1)) == 0 && q > 0) {
+            if ((q & (kBremGroup - 1)) == 0 && q > 0) {
 #pragma unroll
                 for (int m = 0; m < BINS; ++m) {
                     acc[m] += (double)part[m];
                     part[m] = 0.0f;
                 }
             }
+            const float plo = s_plo[q], phi = s_phi[q], pmid = s_pmid[q], dp = s_dp[q];
+            if (kOrdered && tile.band) {
+                const float x = s_T[q], wL = s_pi[q];
+#pragma unroll
+                for (int m = 0; m < BINS; ++m) {
+                    float v = g[m][kBremDeg];
+#pragma unroll
+                    for (int i = kBremDeg - 1; i >= 0; --i) v = fmaf(v, x, g[m][i]);
+                    v *= wL;
+                    const float d = dp * mu[m];  // the escape as below
+                    if (d > 1.0f) {
+                        v *= fast_rcp(d);
+                        part[m] = fmaf(v, fast_exp2(-plo * mu2[m]) - fast_exp2(-phi * mu2[m]), part[m]);
+                    } else {
+                        const float x2 = 0.25f * d * d;
+                        v *= fmaf(x2, fmaf(x2, fmaf(x2, 1.0f / 5040, 1.0f / 120), 1.0f / 6), 1.0f);
+                        part[m] = fmaf(v, fast_exp2(-pmid * mu2[m]), part[m]);
+                    }
+                }
+                continue;
+            }
             // a zero-weight row (a copy that does not carry this tally) adds nothing
             if (!s_live[q]) continue;
             const float T = s_T[q], pi_ = s_pi[q];
-            const float plo = s_plo[q], phi = s_phi[q], pmid = s_pmid[q], dp = s_dp[q];
 #pragma unroll
             for (int m = 0; m < BINS; ++m) {
                 const float Tf = T - keV[m];
@@ -481,7 +757,6 @@ __global__ void __launch_bounds__(kRedThreads) brem_kernel(hr_brem_args p, doubl
         }
 #pragma unroll
         for (int m = 0; m < BINS; ++m) acc[m] += (double)part[m];
-        __syncthreads();
     }
     double *out = partial + (int64_t)blockIdx.x * p.n_E;
 #pragma unroll
@@ -792,6 +1067,47 @@ hr_status dense_plan(int64_t n_items, int64_t tile, int64_t n_E, DensePlan &P) {
     return HR_OK;
 }
 
+// Launch shape and workspace of the brem reduction: bins per thread to the grid
+// (a 201-bin grid takes one, not four), tiles of a power of two rows, at least 32,
+// that make up to 16 blocks per CU (rows below the bins' energies cost less than
+// others, direct ones more), and the class order where it pays.
+constexpr int kBremWaves = 512;  // of the sort, at most
+struct BremPlan {
+    int bins = 4;
+    int64_t rows = 32, gx = 1, windows = 1, waves = 0, per = 0;  // waves: of the sort, 0 none
+    size_t partials = 0, bytes = 0;
+};
+hr_status brem_plan(int64_t n_seg, int64_t n_E, BremPlan &P) {
+    int cu = 0;
+    hr_status st = device_cu(cu);
+    if (st != HR_OK) return st;
+    P.bins = n_E <= kRedThreads ? 1 : (n_E <= 2 * kRedThreads ? 2 : 4);
+    P.windows = (n_E + kRedThreads * P.bins - 1) / (kRedThreads * P.bins);
+    int64_t room = 16 * (int64_t)cu / (P.windows > 0 ? P.windows : 1);
+    room = room < 1 ? 1 : room;
+    while (n_seg > room * P.rows) P.rows *= 2;
+    P.gx = (n_seg + P.rows - 1) / P.rows;
+    // sizes at their bounds, so that a workspace serves fewer rows too
+    const bool some = n_seg > 0 && n_E > 0;
+    int64_t rows_max = (n_seg + 31) / 32 < room ? (n_seg + 31) / 32 : room;
+    // row indices of the order are 32-bit, and so is the laying grid
+    if (some && n_seg <= INT32_MAX && n_E <= (1 << 24) && n_seg >= kBremSortCells / n_E) {
+        P.per = (n_seg + kBremWaves - 1) / kBremWaves;
+        P.per = P.per < 256 ? 256 : (P.per + 63) / 64 * 64;
+        P.waves = (n_seg + P.per - 1) / P.per;
+        P.gx += kBremClasses - 1;  // every class may end in a tile of its own
+        rows_max += kBremClasses - 1;
+    }
+    P.partials = some ? partial_bytes(rows_max, n_E) : 0;
+    P.bytes = P.partials;
+    if (P.waves > 0) {
+        // [partial rows | order | counts | totals | polynomials]
+        P.bytes += (size_t)(n_seg + (kBremWaves + 1) * kBremClasses) * sizeof(uint32_t) +
+                   (size_t)kBremClasses * kBremNodes * (size_t)n_E * sizeof(float);
+    }
+    return HR_OK;
+}
+
 // Launch shape of the uniform-grid reduction.  The window of 64 `bins` bins is
 // the smallest cover of the grid in windows of 256 to 1024 bins, a window's
 // fixed cost per line counted as three bins per lane (the sine and cosine at the
@@ -997,8 +1313,8 @@ extern "C" hr_status hr_brem_workspace_bytes(const hr_brem_args *args, size_t *b
     using namespace hr;
     HR_REQUIRE(args != nullptr && bytes != nullptr, "hr_brem_workspace_bytes: null argument");
     HR_REQUIRE(args->n_seg >= 0 && args->n_E >= 0, "hr_brem_workspace_bytes: negative size");
-    DensePlan P;
-    hr_status st = dense_plan(args->n_seg, kBremTile, args->n_E, P);
+    BremPlan P;
+    hr_status st = brem_plan(args->n_seg, args->n_E, P);
     if (st != HR_OK) return st;
     *bytes = P.bytes;
     return HR_OK;
@@ -1014,23 +1330,49 @@ extern "C" hr_status hr_brem_reduce(const hr_brem_args *args, void *stream) {
     if (p.n_seg == 0 || p.n_E == 0) return HR_OK;
     HR_REQUIRE(p.r_mid && p.v_hat && p.L && p.E_keV && p.E_grid_eV && p.mu && p.out,
                "hr_brem_reduce: null pointer");
-    constexpr int BINS = kDenseBins;
-    DensePlan P;
-    hr_status st = dense_plan(p.n_seg, kBremTile, p.n_E, P);
+    BremPlan P;
+    hr_status st = brem_plan(p.n_seg, p.n_E, P);
     if (st != HR_OK) return st;
     HR_REQUIRE_WS(p.ws, P.bytes, "hr_brem_reduce");
-    const int64_t gx = P.gx;
-    void *ws = p.ws.ptr;
     hipStream_t s = (hipStream_t)stream;
-    const dim3 grid((unsigned)gx, (unsigned)P.bin_tiles);
-    switch (p.n_el) {
-    case 1: hipLaunchKernelGGL((brem_kernel<BINS, 1>), grid, dim3(kRedThreads), 0, s, p, (double *)ws); break;
-    case 2: hipLaunchKernelGGL((brem_kernel<BINS, 2>), grid, dim3(kRedThreads), 0, s, p, (double *)ws); break;
-    case 3: hipLaunchKernelGGL((brem_kernel<BINS, 3>), grid, dim3(kRedThreads), 0, s, p, (double *)ws); break;
-    default: hipLaunchKernelGGL((brem_kernel<BINS, 4>), grid, dim3(kRedThreads), 0, s, p, (double *)ws); break;
+    double *ws = (double *)p.ws.ptr;
+    BremOrder o{};
+    if (P.waves > 0) {
+        uint32_t *order = (uint32_t *)((char *)p.ws.ptr + P.partials), *counts = order + p.n_seg;
+        uint32_t *totals = counts + P.waves * kBremClasses;
+        float *poly = (float *)(totals + kBremClasses);
+        o = BremOrder{order, totals, poly};
+        hipLaunchKernelGGL(brem_count_kernel, dim3((unsigned)P.waves), dim3(64), 0, s, p, P.per, counts);
+        HR_CHECK_HIP(hipGetLastError());
+        hipLaunchKernelGGL(brem_scan_kernel, dim3(kBremClasses), dim3(64), 0, s, counts, P.waves, totals);
+        HR_CHECK_HIP(hipGetLastError());
+        const int64_t groups = (p.n_E + kBremPolyBins - 1) / kBremPolyBins;
+        hipLaunchKernelGGL(brem_lay_kernel, dim3((unsigned)(P.waves + groups * kBremClasses)), dim3(64), 0, s, p, P.per,
+                           P.waves, counts, totals, order, poly);
+        HR_CHECK_HIP(hipGetLastError());
     }
+    const dim3 grid((unsigned)P.gx, (unsigned)P.windows);
+#define HR_BREM(B, NEL)                                                                                             \
+    if (P.waves > 0)                                                                                                \
+        hipLaunchKernelGGL((brem_kernel<B, NEL, true>), grid, dim3(kRedThreads), 0, s, p, P.rows, o, ws);           \
+    else                                                                                                            \
+        hipLaunchKernelGGL((brem_kernel<B, NEL, false>), grid, dim3(kRedThreads), 0, s, p, P.rows, o, ws)
+#define HR_BREM_EL(B)                    \
+    switch (p.n_el) {                    \
+    case 1: HR_BREM(B, 1); break;        \
+    case 2: HR_BREM(B, 2); break;        \
+    case 3: HR_BREM(B, 3); break;        \
+    default: HR_BREM(B, 4); break;       \
+    }
+    switch (P.bins) {
+    case 1: HR_BREM_EL(1); break;
+    case 2: HR_BREM_EL(2); break;
+    default: HR_BREM_EL(4); break;
+    }
+#undef HR_BREM_EL
+#undef HR_BREM
     HR_CHECK_HIP(hipGetLastError());
-    return row_sum((const double *)ws, gx, p.n_E, p.out, s);
+    return row_sum(ws, P.gx, p.n_E, p.out, s);
 }
 
 namespace hr {
