@@ -996,40 +996,68 @@ __global__ void __launch_bounds__(256) window_sum_kernel(const double *__restric
 }
 
 // out[d][e] += spec[d][e] + sum_q tail(dep[d][.][q], (e - (q - n)) dE) over node slots q in [q_lo, q_hi).
-constexpr int kConvTile = 256;
-__global__ void __launch_bounds__(kConvTile) window_tail_kernel(const double *__restrict__ spec,
-                                                                const double *__restrict__ dep, int64_t n,
-                                                                double dE, int64_t q_lo, int64_t q_hi,
-                                                                double *__restrict__ out) {
-    __shared__ double s_m[3][kConvTile];
-    __shared__ double s_inv[2 * kConvTile];
+// FP64-bound: four operations a cell.  A block covers kConvTile bins, four
+// neighbours to a lane, and its four waves a quarter of each tile of nodes: the
+// reciprocals of a lane's bins slide along with the nodes, so that four nodes
+// cost 4 reads of reciprocals (kept by index mod 4: no bank conflict) and 8 of
+// moments for 16 cells, where one bin a thread read 4 values for each and was
+// bound by LDS (64 directions x 4,096 bins: 488 us, 220 so).
+constexpr int kConvTile = 256, kConvWaves = 4;
+__global__ void __launch_bounds__(64 * kConvWaves) window_tail_kernel(const double *__restrict__ spec,
+                                                                      const double *__restrict__ dep, int64_t n,
+                                                                      double dE, int64_t q_lo, int64_t q_hi,
+                                                                      double *__restrict__ out) {
+    static_assert(kConvTile == 64 * kConvWaves && kConvWaves == 4, "four bins to a lane, a node to a thread");
+    __shared__ double4 s_m[kConvTile];
+    // reciprocal of bin x node offset o = (e0 - q0 + n) + k - 255 at [k % 4][k / 4]
+    __shared__ double s_inv[4][2 * kConvTile / 4];
+    __shared__ double s_sum[kConvWaves][kConvTile];
     const int d = blockIdx.y;
     const int64_t e0 = (int64_t)blockIdx.x * kConvTile;
-    const int t = threadIdx.x;
-    const int64_t e = e0 + t;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const double *D = dep + (int64_t)d * 9 * n;
     const int64_t L = 3 * n;
-    double acc = 0.0;
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
     for (int64_t q0 = q_lo; q0 < q_hi; q0 += kConvTile) {
         const int64_t q = q0 + t;
         const bool in = q < q_hi;
-        s_m[0][t] = in ? D[q] : 0.0;
-        s_m[1][t] = in ? D[L + q] : 0.0;
-        s_m[2][t] = in ? D[2 * L + q] : 0.0;
-        // offsets e - (q - n) over the tile: o = (e0 - q0 + n) + (t_e - t_q), t_e - t_q in [-255, 255]
+        __syncthreads();
+        s_m[t] = in ? make_double4(D[q], D[L + q], D[2 * L + q], 0.0) : make_double4(0.0, 0.0, 0.0, 0.0);
         for (int k = t; k < 2 * kConvTile; k += kConvTile) {
             const int64_t o = (e0 - q0 + n) + (int64_t)(k - (kConvTile - 1));
-            s_inv[k] = o == 0 ? 0.0 : 1.0 / ((double)o * dE);
+            s_inv[k & 3][k >> 2] = o == 0 ? 0.0 : rcp_nr((double)o * dE);
         }
         __syncthreads();
-        const int m = q_hi - q0 < kConvTile ? (int)(q_hi - q0) : kConvTile;
-        for (int j = 0; j < m; ++j) {
-            const double inv = s_inv[t - j + (kConvTile - 1)];
-            acc += (s_m[0][j] + (s_m[1][j] + s_m[2][j] * inv) * inv) * inv * inv;
+        // bin e0 + 4 lane + m against node q0 + 4 i + r: k = 4 (lane - i + 63) + (m - r + 3)
+        const int i0 = wave * (kConvTile / 4 / kConvWaves);
+        double v[7];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) v[k] = s_inv[k][lane - i0 + 64];
+#pragma unroll 2
+        for (int i = i0; i < i0 + kConvTile / 4 / kConvWaves; ++i) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) v[k + 4] = v[k];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[k] = s_inv[k][lane - i + 63];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const double4 M = s_m[4 * i + r];
+#pragma unroll
+                for (int m = 0; m < 4; ++m) {
+                    const double inv = v[m - r + 3];
+                    acc[m] = fma(fma(fma(M.z, inv, M.y), inv, M.x), inv * inv, acc[m]);
+                }
+            }
         }
-        __syncthreads();
     }
-    if (e < n) out[(int64_t)d * n + e] += spec[(int64_t)d * n + e] + acc;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) s_sum[wave][4 * lane + m] = acc[m];
+    __syncthreads();
+    const int64_t e = e0 + t;
+    if (e >= n) return;
+    double sum = 0.0;
+    for (int w = 0; w < kConvWaves; ++w) sum += s_sum[w][t];
+    out[(int64_t)d * n + e] += spec[(int64_t)d * n + e] + sum;
 }
 
 __global__ void fill_zero_kernel(double *__restrict__ p, int64_t n) {
