@@ -146,7 +146,7 @@ __device__ __forceinline__ void sincos_turns(double u, float &s, float &c) {
 }
 
 constexpr int kFieldThreads = 256;
-constexpr int kFieldTile = 256;
+constexpr int kFieldTile = 128;  // 64 and 224 measured 4 % slower on the case of the grouped kernel
 constexpr int kFieldGroup = 8;  // lines summed in FP32 before each FP64 add
 
 // Line constants staged in LDS: FP64 terms of the two phases (in turns); FP32
@@ -188,17 +188,17 @@ __device__ __forceinline__ void stage_line(FieldTile &T, const double *__restric
         T.flag[tid] = live ? ((float)q * (float)q < kSeriesW2 ? 2 : 1) : 0;
 }
 
-// One (line l, bin m) cell added to the FP32 group sums.
-template <bool kSeries, int BINS>
+// The cells of line l in the first N of the thread's bins, added to the FP32 group sums.
+template <bool kSeries, int N, int BINS>
 __device__ __forceinline__ void field_cell(const FieldTile &T, int l, const double (&E)[BINS],
-                                           const double (&D)[BINS], float (&g)[BINS][4]) {
+                                           const double (&D)[BINS], float (&g)[N][4]) {
     const double a_t = T.a_t[l], aEc_t = T.aEc_t[l], hdL_t = T.hdL_t[l];
     const double ps_t = T.ps_t[l], gp_t = T.gp_t[l], Le_t = T.Le_t[l];
     const float csr = T.c[0][l], csi = T.c[1][l], cpr = T.c[2][l], cpi = T.c[3][l];
     const float h_apb = T.h_apb[l], h_bma = T.h_bma[l], h_qapb = T.h_qapb[l], h_qbma = T.h_qbma[l];
     const float q = T.q[l], qq = q * q;
 #pragma unroll
-    for (int m = 0; m < BINS; ++m) {
+    for (int m = 0; m < N; ++m) {
         const double uv = fma(-hdL_t, D[m], fma(a_t, E[m], -aEc_t));
         const double uph = fma(-Le_t, D[m], fma(ps_t, E[m], -gp_t));
         float sv, cv, sp, cp;
@@ -222,30 +222,56 @@ __device__ __forceinline__ void field_cell(const FieldTile &T, int l, const doub
     }
 }
 
-// acc += the fields of tile lines [first, nt), in FP32 groups of kFieldGroup lines.
-template <int BINS>
-__device__ __forceinline__ void tile_fields(const FieldTile &T, int first, int nt, const double (&E)[BINS],
-                                            const double (&D)[BINS], double (&acc)[BINS][4]) {
+// acc += the fields of tile lines [first, nt) in the first N bins, in FP32 groups of
+// kFieldGroup lines.
+template <int N, int BINS>
+__device__ __forceinline__ void tile_runs(const FieldTile &T, int first, int nt, const double (&E)[BINS],
+                                          const double (&D)[BINS], double (&acc)[BINS][4]) {
     for (int l0 = first; l0 < nt; l0 += kFieldGroup) {
-        float g[BINS][4];
+        float g[N][4];
 #pragma unroll
-        for (int m = 0; m < BINS; ++m)
+        for (int m = 0; m < N; ++m)
 #pragma unroll
             for (int c = 0; c < 4; ++c) g[m][c] = 0.0f;
         const int l1 = l0 + kFieldGroup < nt ? l0 + kFieldGroup : nt;
         for (int l = l0; l < l1; ++l) {
             const int f = T.flag[l];  // uniform over the block
-            if (f == 1) field_cell<false, BINS>(T, l, E, D, g);
-            else if (f == 2) field_cell<true, BINS>(T, l, E, D, g);
+            if (f == 1) field_cell<false, N, BINS>(T, l, E, D, g);
+            else if (f == 2) field_cell<true, N, BINS>(T, l, E, D, g);
         }
 #pragma unroll
-        for (int m = 0; m < BINS; ++m)
+        for (int m = 0; m < N; ++m)
 #pragma unroll
             for (int c = 0; c < 4; ++c) acc[m][c] += (double)g[m][c];
     }
 }
 
-// Block (split s, row r, bin window w): lines of row r in tiles s, s+S, ...;
+// A thread has bins tid + 256 m of its window; of a grid that ends within, each wave
+// evaluates only the `runs` of 64 bins that it has.  Call from rows to spectrum, all
+// bins evaluated (and fields split by whole tiles of 256 lines) and now: 81,000 lines
+// x 4 rows x 300 bins with the grouped term 535 -> 346 us, 10,000 lines x 4 x 300
+// without 214 -> 97 us, 1,000 x 9 x 600 233 -> 115 us.
+template <bool kWhole, int BINS>
+__device__ __forceinline__ void tile_fields(const FieldTile &T, int first, int nt, int runs, const double (&E)[BINS],
+                                            const double (&D)[BINS], double (&acc)[BINS][4]) {
+    static_assert(BINS == 4, "the cases below");
+    if (kWhole) return tile_runs<4>(T, first, nt, E, D, acc);
+    switch (runs) {
+    case 4: tile_runs<4>(T, first, nt, E, D, acc); break;
+    case 3: tile_runs<3>(T, first, nt, E, D, acc); break;
+    case 2: tile_runs<2>(T, first, nt, E, D, acc); break;
+    case 1: tile_runs<1>(T, first, nt, E, D, acc); break;
+    default: break;
+    }
+}
+
+__device__ __forceinline__ int wave_runs(int64_t n_E, int win, int bins) {
+    const int64_t left = n_E - (int64_t)win * bins * kFieldThreads - (threadIdx.x & ~63);
+    const int64_t runs = left > 0 ? (left + kFieldThreads - 1) / kFieldThreads : 0;
+    return __builtin_amdgcn_readfirstlane((int)(runs < bins ? runs : bins));
+}
+
+// Block (split s, row r, bin window w): lines [n s / S, n (s+1) / S) of row r;
 // thread t owns bins w*256*BINS + t + 256*m.  Writes its partial field
 // (or adds it when S == 1).
 template <int BINS>
@@ -272,14 +298,14 @@ __global__ void __launch_bounds__(kFieldThreads) coherent_field_kernel(hr_cohere
         for (int c = 0; c < 4; ++c) acc[m][c] = 0.0;
     const int64_t plane = (int64_t)p.n_rows * p.ld;
     const double *R = p.rec + (int64_t)row * p.ld;
-    const int64_t n_tiles = (p.n_lines + kFieldTile - 1) / kFieldTile;
-    for (int64_t tile = split; tile < n_tiles; tile += S) {
-        const int64_t j0 = tile * kFieldTile;
-        const int nt = (int)(p.n_lines - j0 < kFieldTile ? p.n_lines - j0 : kFieldTile);
+    const int runs = wave_runs(n_E, win, BINS);
+    const int64_t end = p.n_lines * (split + 1) / S;
+    for (int64_t j0 = p.n_lines * split / S; j0 < end; j0 += kFieldTile) {
+        const int nt = (int)(end - j0 < kFieldTile ? end - j0 : kFieldTile);
         __syncthreads();
         if (tid < nt) stage_line(T, R, plane, j0 + tid, tid);
         __syncthreads();
-        tile_fields<BINS>(T, 0, nt, E, D, acc);
+        tile_fields<false, BINS>(T, 0, nt, runs, E, D, acc);
     }
 #pragma unroll
     for (int m = 0; m < BINS; ++m) {
@@ -302,13 +328,19 @@ __global__ void __launch_bounds__(kFieldThreads) coherent_field_kernel(hr_cohere
 // lines: one evaluation of each cell serves both (81,000 lines x 4 rows x 1,024
 // bins: 340 us flat and 404 us grouped as two launches; the call from rows to
 // blended spectrum 845 us so, 526 us with one).
-template <int BINS, bool kField>
-__global__ void __launch_bounds__(kFieldThreads) coherent_grouped_kernel(hr_coherent_field_args p,
+template <int BINS, bool kField, bool kWhole>
+__global__ void __launch_bounds__(kFieldThreads, 3) coherent_grouped_kernel(hr_coherent_field_args p,
                                                                          const int64_t *__restrict__ gs,
                                                                          int64_t n_groups, int W, int S,
                                                                          double *__restrict__ out,
                                                                          double *__restrict__ field) {
     __shared__ FieldTile T;
+    // the thread's flat fields, in registers on whole windows only: beside the cases of
+    // a partial one they leave two waves to a SIMD instead of three (4,001 histories x
+    // 1,024 bins: 541 us the call in registers, 562 in LDS, 551 with two waves).
+    constexpr bool kShared = kField && !kWhole;
+    __shared__ double s_flat[kShared ? BINS * 4 : 1][kShared ? kFieldThreads : 1];
+    double flat[kField && kWhole ? BINS : 1][4];
     const int tid = threadIdx.x;
     const int row = (int)(blockIdx.y / W), win = (int)(blockIdx.y % W);
     const int split = (int)blockIdx.x;
@@ -322,12 +354,16 @@ __global__ void __launch_bounds__(kFieldThreads) coherent_grouped_kernel(hr_cohe
         E[m] = valid[m] ? p.E_grid[k] : 0.0;
         D[m] = valid[m] ? p.dom[k] : 0.0;
     }
-    double G[BINS], acc[BINS][4], flat[BINS][4];
+    double G[BINS], acc[BINS][4];
 #pragma unroll
     for (int m = 0; m < BINS; ++m) {
         G[m] = 0.0;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) acc[m][c] = flat[m][c] = 0.0;
+        for (int c = 0; c < 4; ++c) {
+            acc[m][c] = 0.0;
+            if constexpr (kShared) s_flat[4 * m + c][tid] = 0.0;
+            else if constexpr (kField) flat[m][c] = 0.0;
+        }
     }
     const int64_t plane = (int64_t)p.n_rows * p.ld;
     const double *R = p.rec + (int64_t)row * p.ld;
@@ -336,6 +372,7 @@ __global__ void __launch_bounds__(kFieldThreads) coherent_grouped_kernel(hr_cohe
         const int64_t c = gs[g];
         return c < 0 ? 0 : (c > p.n_lines ? p.n_lines : c);
     };
+    const int runs = wave_runs(n_E, win, BINS);
     int64_t grp = g_lo, closes = column(grp + 1 <= n_groups ? grp + 1 : n_groups);
     const int64_t end = column(g_hi);
     for (int64_t t0 = column(g_lo); t0 < end; t0 += kFieldTile) {
@@ -346,7 +383,7 @@ __global__ void __launch_bounds__(kFieldThreads) coherent_grouped_kernel(hr_cohe
         for (int l = 0; l < nt;) {
             int stop = nt;
             if (closes - t0 < nt) stop = closes - t0 > l ? (int)(closes - t0) : l;
-            tile_fields<BINS>(T, l, stop, E, D, acc);
+            tile_fields<kWhole, BINS>(T, l, stop, runs, E, D, acc);
             l = stop;
             while (grp < g_hi && closes <= t0 + l) {
 #pragma unroll
@@ -355,7 +392,8 @@ __global__ void __launch_bounds__(kFieldThreads) coherent_grouped_kernel(hr_cohe
                             acc[m][3] * acc[m][3];
 #pragma unroll
                     for (int c = 0; c < 4; ++c) {
-                        if (kField) flat[m][c] += acc[m][c];
+                        if constexpr (kShared) s_flat[4 * m + c][tid] += acc[m][c];
+                        else if constexpr (kField) flat[m][c] += acc[m][c];
                         acc[m][c] = 0.0;
                     }
                 }
@@ -373,8 +411,11 @@ __global__ void __launch_bounds__(kFieldThreads) coherent_grouped_kernel(hr_cohe
         if constexpr (kField) {
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                if (S == 1) field[((int64_t)row * 4 + c) * n_E + k] += flat[m][c];
-                else field[(((int64_t)split * p.n_rows + row) * 4 + c) * n_E + k] = flat[m][c];
+                double f;
+                if constexpr (kShared) f = s_flat[4 * m + c][tid];
+                else f = flat[m][c];
+                if (S == 1) field[((int64_t)row * 4 + c) * n_E + k] += f;
+                else field[(((int64_t)split * p.n_rows + row) * 4 + c) * n_E + k] = f;
             }
         }
     }
@@ -428,11 +469,19 @@ __global__ void __launch_bounds__(256) coherent_blend_kernel(const double *__res
 }
 
 constexpr int kFieldBins = 4;
+
+// Whether every wave of every window has all its runs of 64 bins (the grouped kernels
+// then drop the other cases).
+bool whole_windows(int64_t n_E) {
+    constexpr int64_t per_block = (int64_t)kFieldThreads * kFieldBins;
+    return (n_E + 63) / 64 * 64 % per_block == 0;
+}
 constexpr size_t kMaxPartialBytes = size_t(1) << 30;
 
 // Launch shape of hr_coherent_field: S splits along the line axis (fill the
-// chip ~8 workgroups per CU, never more than there are tiles, partials under
-// kMaxPartialBytes) over n_rows*W row windows; workspace bytes for S > 1.
+// chip ~8 workgroups per CU, of a whole tile each beyond the 3 that a CU holds
+// and of 32 lines up to there, partials under kMaxPartialBytes) over n_rows*W row
+// windows; workspace bytes for S > 1.
 struct FieldPlan {
     int64_t W = 0, S = 1;
     size_t bytes = 0;
@@ -445,9 +494,11 @@ hr_status field_plan(const hr_coherent_field_args &p, FieldPlan &P) {
     P.W = (p.n_E + per_block - 1) / per_block;
     const int64_t n_tiles = (p.n_lines + kFieldTile - 1) / kFieldTile;
     const int64_t cells = (int64_t)p.n_rows * 4 * p.n_E;
-    int64_t S = (int64_t)cu * 8 / ((int64_t)p.n_rows * P.W);
+    const int64_t blocks = (int64_t)p.n_rows * P.W, chunks = (p.n_lines + 31) / 32;
+    int64_t S = chunks < (int64_t)cu * 3 / blocks ? chunks : (int64_t)cu * 3 / blocks;
+    if (S < n_tiles) S = n_tiles;
+    if (S > (int64_t)cu * 8 / blocks) S = (int64_t)cu * 8 / blocks;
     if (S < 1) S = 1;
-    if (S > n_tiles) S = n_tiles;
     const int64_t s_cap = (int64_t)(kMaxPartialBytes / ((size_t)cells * sizeof(double)));
     if (S > s_cap) S = s_cap > 1 ? s_cap : 1;
     if (S < 1) S = 1;
@@ -500,12 +551,14 @@ hr_status grouped_run(const hr_coherent_grouped_args *args, bool field, const ch
     double *ws = (double *)p.ws.ptr;
     double *out = S > 1 ? ws : args->grouped, *flat = S > 1 ? ws + S * cells : p.field;
     const dim3 grid((unsigned)S, (unsigned)(p.n_rows * W));
-    if (field)
-        hipLaunchKernelGGL((coherent_grouped_kernel<kFieldBins, true>), grid, dim3(kFieldThreads), 0, s, p,
-                           args->group_start, n_groups, (int)W, (int)S, out, flat);
-    else
-        hipLaunchKernelGGL((coherent_grouped_kernel<kFieldBins, false>), grid, dim3(kFieldThreads), 0, s, p,
-                           args->group_start, n_groups, (int)W, (int)S, out, nullptr);
+#define HR_GROUPED(FIELD, WHOLE)                                                                                       \
+    hipLaunchKernelGGL((coherent_grouped_kernel<kFieldBins, FIELD, WHOLE>), grid, dim3(kFieldThreads), 0, s, p,        \
+                       args->group_start, n_groups, (int)W, (int)S, out, flat)
+    if (field && whole_windows(p.n_E)) HR_GROUPED(true, true);
+    else if (field) HR_GROUPED(true, false);
+    else if (whole_windows(p.n_E)) HR_GROUPED(false, true);
+    else HR_GROUPED(false, false);
+#undef HR_GROUPED
     HR_CHECK_HIP(hipGetLastError());
     if (S == 1) return HR_OK;
     st = row_sum(out, S, cells, args->grouped, s);

@@ -1,6 +1,6 @@
 """Flat field and grouped term in one pass against the two separate ones (GPU).
 
-Groups of no, one and many lines, ends on and beside the 256 lines a block stages
+Groups of no, one and many lines, ends on and beside the 128 lines a block stages
 and the 8 it sums in FP32, one chunk and many.  Both routes sum the same FP32
 cells, in FP32 groups of at most 8 that start elsewhere: they may differ by the
 bound the field test uses on either (2e-6 of the lines' L1 size), and the grouped
@@ -14,13 +14,13 @@ pytestmark = pytest.mark.gpu
 SIZES = {
     "one_line": [1],
     "empty_groups": [0, 0, 3, 0, 5, 0],
-    "tile_edges": [255, 1, 256, 257, 1, 7, 8, 9],
+    "tile_edges": [127, 1, 128, 129, 255, 256, 257, 1, 7, 8, 9],
     "one_long": [1500],
     "histories": None,
 }
 
 
-@pytest.mark.parametrize("n_E", [5, 1100])
+@pytest.mark.parametrize("n_E", [5, 300, 1100])
 @pytest.mark.parametrize("sizes", list(SIZES))
 def test_one_pass_equals_two(device, sizes, n_E):
     import torch
