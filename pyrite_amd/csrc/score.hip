@@ -118,12 +118,15 @@ constexpr int kSincGroup = 4;   // cells summed in FP32 before each FP64 add (al
 // sine and cosine at the middle of its run and steps outward both ways (at most
 // BINS/2 steps: the sines stay within 1e-13).  The divisor is the distance in
 // bins, d = (k - n) + u(n)/du with n the bin nearest the centre, so it is exact to
-// FP32 rounding there; sqrt(w)/(pi du) rides on the sines.
+// FP32 rounding there; 1/(pi du) rides on the sines.  The weight multiplies the
+// square on its own and FP32 groups end with every eighth line of the input, so that
+// weighted copies add up to the unweighted sum (a weight of 2 is twice the line).
 //
 // VALU bound: about 31 SIMD cycles per cell (FP64, conversions and selects issue
 // in 4, plain FP32 in 2, the reciprocal in 8) against 52 of a cell with its own
-// phase.  2.7e6 lines (half live) on 1024 bins: 608 us before, 402 now
-// (about 49 cycles: staging, FP64 sums and waves of uneven work make the rest).
+// phase.  2.7e6 lines (1.07e6 live) on 1024 bins: 608 us before, 441 now
+// (about 54 cycles: staging, FP64 sums and waves of uneven work make the rest; 402
+// with sqrt(w) on the sines and groups across the input's eighths).
 constexpr int kSincWaves = 4;     // waves per block, each with its own lines
 constexpr int kSincBlock = 64 * kSincWaves;
 constexpr int kSincChunk = 64;    // lines a wave stages at a time (one per lane)
@@ -147,7 +150,7 @@ __device__ __forceinline__ double horner(const double (&c)[N], double z) {
 struct alignas(16) SincLine {
     double u0, du;    // u = u0 + k du, turns of pi
     double cd, sd;    // cos, sin of pi du
-    double q;         // sqrt(w) / (pi du)
+    double q;         // 1 / (pi du)
     float nf, f, w;   // n - bin0 for the integer n nearest the centre; u(n)/du; w
     int direct;       // no recurrence: see the staging
 };
@@ -199,7 +202,7 @@ __global__ void __launch_bounds__(kSincBlock, 4) sincsq_uniform_kernel(
             o.du = al * dE;
             sincospi(o.du - 2.0 * rint(0.5 * o.du), &o.sd, &o.cd);
             const double inv_du = rcp_nr(o.du);
-            o.q = sqrt_nr((double)wl) * inv_pi * inv_du;
+            o.q = inv_pi * inv_du;
             const double n = rint((er - E0) * inv_dE), u = fma(n, o.du, o.u0);
             o.nf = (float)(n - (double)bin0);
             o.f = (float)(u * inv_du);
@@ -208,19 +211,20 @@ __global__ void __launch_bounds__(kSincBlock, 4) sincsq_uniform_kernel(
             // off by up to 1e-13 of the largest of the run, min(1, 8 pi du), and by
             // the rounding of its phase, 1e-15 du: below 3e-8 of itself unless
             // |u(n)| is under this line, where every cell is taken on its own
-            // (1 line in 1e4 at most).  So are negative weights and steps too
-            // small to divide by.
+            // (1 line in 1e4 at most).  So are steps too small to divide by.
             const double small = 4.0e-6 * fmin(1.0, 25.0 * fabs(o.du)) + 4.0e-8 * fabs(o.du);
-            o.direct = !(fabs(o.du) >= 1.0e-250) || wl < 0.0f || !(fabs(u) >= small);
+            o.direct = !(fabs(o.du) >= 1.0e-250) || !(fabs(u) >= small);
             lines[__popcll(live & ((1ULL << lane) - 1ULL))] = o;
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        for (int j0 = 0; j0 < n_live; j0 += kSincGroup) {
+        uint64_t left = live;  // from the eighth line that `stop` belongs to on
+        for (int j0 = 0, stop = 0; j0 < n_live;) {
+            for (; stop <= j0; left >>= 8) stop += __popcll(left & 0xff);
             float g[BINS];
 #pragma unroll
             for (int m = 0; m < BINS; ++m) g[m] = 0.0f;
-            const int j1 = j0 + kSincGroup < n_live ? j0 + kSincGroup : n_live;
+            const int j1 = j0 + kSincGroup < stop ? j0 + kSincGroup : stop;
 #pragma unroll 2
             for (int j = j0; j < j1; ++j) {
                 const SincLine &o = lines[j];
@@ -235,6 +239,7 @@ __global__ void __launch_bounds__(kSincBlock, 4) sincsq_uniform_kernel(
                     continue;
                 }
                 const double cd = o.cd, c2 = 2.0 * cd, q = o.q;
+                const float wl = o.w;
                 const double u = fma(kb, o.du, o.u0), r = u - rint(u), z = r * r;
                 const double S = (q * r) * horner(sin_r, z), C = q * horner(cos_r, z);
                 const float base = run0f - o.nf, f = o.f;
@@ -245,8 +250,8 @@ __global__ void __launch_bounds__(kSincBlock, 4) sincsq_uniform_kernel(
                     const int mu = kMid + i, ml = kMid - 1 - i;
                     const float xu = (float)up * __builtin_amdgcn_rcpf((base + (float)mu) + f);
                     const float xl = (float)lo * __builtin_amdgcn_rcpf((base + (float)ml) + f);
-                    g[mu] = fmaf(xu, xu, g[mu]);
-                    g[ml] = fmaf(xl, xl, g[ml]);
+                    g[mu] = fmaf(wl * xu, xu, g[mu]);
+                    g[ml] = fmaf(wl * xl, xl, g[ml]);
                     const double un = fma(c2, up, -up_p), ln = fma(c2, lo, -lo_p);
                     up_p = up;
                     up = un;
@@ -256,6 +261,7 @@ __global__ void __launch_bounds__(kSincBlock, 4) sincsq_uniform_kernel(
             }
 #pragma unroll
             for (int m = 0; m < BINS; ++m) acc[m] += (double)g[m];
+            j0 = j1;
         }
     }
     // the block's partial row: its waves added in order
@@ -1168,7 +1174,8 @@ hr_status brem_plan(int64_t n_seg, int64_t n_E, BremPlan &P) {
 // of `per` lines, 64 where that leaves every resident wave four, fewer on small
 // inputs so that all of them work.  Dead lines come in runs, so where chunks
 // abound four times the resident blocks are launched to even the waves out
-// (2.7e6 lines on 1024 bins: 448 us resident, 402 so; 1.8e5 lines lose 20 us).
+// (2.7e6 lines on 1024 bins, the weight still on the sines: 448 us resident, 402
+// so; 1.8e5 lines lose 20 us).
 struct SincPlan {
     int bins = 16, per = kSincChunk;
     int64_t gx = 1, windows = 1;
