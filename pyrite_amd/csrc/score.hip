@@ -907,8 +907,8 @@ __device__ __forceinline__ void window_moments(WindowShared &sh, double *__restr
 // Deposits one line per lane (w == 0: none); every lane of the wave takes part.
 // A window's length goes as 1/L: most lines cover a few bins, one in hundreds the
 // whole grid, and a lane that walked its own held the other 63 up (12,007
-// segments x 64 reflections x 64 rays: 5.6 to 35 ms by the draw of lengths, 2.2
-// to 2.4 so).  Windows of up to kOwnCells bins stay with their lane; longer ones
+// segments x 64 reflections x 64 rays: 5.6 to 35 ms by the draw of lengths, 1.9
+// to 2.1 so).  Windows of up to kOwnCells bins stay with their lane; longer ones
 // go through the wave's queue, four at a time to 16 lanes each, and those above
 // kGroupCells to the whole wave.
 constexpr int kOwnCells = 8, kGroupCells = 128, kGroupLanes = 16;
