@@ -327,7 +327,7 @@ __global__ void __launch_bounds__(kFieldThreads) coherent_field_kernel(hr_cohere
 // With kField the groups' fields are added up too, the flat field of the same
 // lines: one evaluation of each cell serves both (81,000 lines x 4 rows x 1,024
 // bins: 340 us flat and 404 us grouped as two launches; the call from rows to
-// blended spectrum 845 us so, 526 us with one).
+// blended spectrum 845 us so, 535 us with one).
 template <int BINS, bool kField, bool kWhole>
 __global__ void __launch_bounds__(kFieldThreads, 3) coherent_grouped_kernel(hr_coherent_field_args p,
                                                                          const int64_t *__restrict__ gs,
