@@ -8,12 +8,14 @@
 //  * the prologue (resonance root, couplings, amplitudes, weights) runs in FP64:
 //    it is once per line, and keeping the resonance energy E_r and the sinc slope
 //    a in FP64 keeps the phase a(E - E_r) exact to ~1e-11 turns;
-//  * the reduction cell evaluates the phase u = a(E - E_r)/pi in FP64 (one FMA
-//    on a uniform grid), reduces it to r = u - rint(u) in FP64, and takes
-//    [sin(pi r) / (pi u)]^2 in FP32 (polynomial sine, hardware reciprocal); cells
-//    are summed in FP32 over groups of 4 lines (all terms are positive) and in
-//    FP64 beyond;
-//  * the brem cell is FP32 (as the reference's), its sums FP64.
+//  * a reduction cell is [sin(pi u) / (pi u)]^2, u = a(E - E_r)/pi.  In general u is
+//    formed in FP64, reduced to r = u - rint(u) in FP64, and the cell taken in FP32
+//    (polynomial sine, hardware reciprocal).  On a uniform grid the sines of lines
+//    without a bin in their central half period |u| < 1/2 are stepped from bin to
+//    bin in FP64 and divided in FP32 by the distance in bins.  Cells are summed in
+//    FP32 over groups of 4 lines (all terms are positive) and in FP64 beyond;
+//  * the brem cell is FP32 (as the reference's), its sums FP64; of large inputs the
+//    cross section is taken from FP32 polynomials that are fitted in FP64.
 // Reductions never use atomics: each workgroup writes a partial spectrum and a
 // second pass adds the partials in a fixed order, so results are bitwise
 // reproducible for a fixed launch shape.
@@ -94,14 +96,24 @@ constexpr float kSinPiOverPi[5] = {1.0f, -1.6449331045150757f, 0.811712443828582
 // central period has u == r, elsewhere |u| >= 1/2), so fminf(x, 1) only trims
 // rounding, and at u == 0 (r == 0) it turns 0 * inf = NaN into the limit 1,
 // where the reference substitutes x = 1e-20.
-__device__ __forceinline__ float sinc2_cell(float r, float uf) {
+__device__ __forceinline__ float sinc_poly(float r) {
     const float r2 = r * r;
     float s = kSinPiOverPi[4];
     s = fmaf(s, r2, kSinPiOverPi[3]);
     s = fmaf(s, r2, kSinPiOverPi[2]);
     s = fmaf(s, r2, kSinPiOverPi[1]);
-    s = fmaf(s, r2, kSinPiOverPi[0]);
-    const float x = fminf(r * __builtin_amdgcn_rcpf(uf) * s, 1.0f);
+    return fmaf(s, r2, kSinPiOverPi[0]);
+}
+__device__ __forceinline__ float sinc2_cell(float r, float uf) {
+    const float x = fminf(r * __builtin_amdgcn_rcpf(uf) * sinc_poly(r), 1.0f);
+    return x * x;
+}
+
+// The same for finite u with r / u = 1 exact where r == u, so that the central half
+// period carries the polynomial's rounding alone (root mean square error of a cell
+// there 4.9e-8 against 7.4e-8).
+__device__ __forceinline__ float sinc2_near(float r, float uf) {
+    const float x = (r == uf ? 1.0f : r * __builtin_amdgcn_rcpf(uf)) * sinc_poly(r);
     return x * x;
 }
 
@@ -124,12 +136,18 @@ constexpr int kSincGroup = 4;   // cells summed in FP32 before each FP64 add (al
 //
 // VALU bound: about 31 SIMD cycles per cell (FP64, conversions and selects issue
 // in 4, plain FP32 in 2, the reciprocal in 8) against 52 of a cell with its own
-// phase.  2.7e6 lines (1.07e6 live) on 1024 bins: 608 us before, 441 now
-// (about 54 cycles: staging, FP64 sums and waves of uneven work make the rest; 402
-// with sqrt(w) on the sines and groups across the input's eighths).
+// phase.  2.7e6 lines of 5 MeV electrons (1.47e6 live) on 1024 bins of 48 eV: 600 us
+// with a phase per cell, 451 so (about 40 cycles: staging, the lines taken cell by
+// cell, FP64 sums and waves of uneven work make the rest).  Lines wider than a bin
+// are all taken cell by cell: 1e6 of them on 1024 bins 523 us before, 513 so.
 constexpr int kSincWaves = 4;     // waves per block, each with its own lines
 constexpr int kSincBlock = 64 * kSincWaves;
 constexpr int kSincChunk = 64;    // lines a wave stages at a time (one per lane)
+
+// Mean relative error of v_rcp_f32, all mantissas with the density of a logarithm
+// (measured; its root mean square is 2.8e-8).  Left in, it would be 1.3e-8 of a sum
+// of many lines.
+constexpr double kRcpMean = -6.4e-9;
 
 // sin(pi r)/r and cos(pi r) on |r| <= 1/2 in r^2 (Chebyshev interpolation of
 // each; errors 1.6e-13 and 2.0e-15).
@@ -150,7 +168,7 @@ __device__ __forceinline__ double horner(const double (&c)[N], double z) {
 struct alignas(16) SincLine {
     double u0, du;    // u = u0 + k du, turns of pi
     double cd, sd;    // cos, sin of pi du
-    double q;         // 1 / (pi du)
+    double q;         // 1 / (pi du), the reciprocal's mean error taken off
     float nf, f, w;   // n - bin0 for the integer n nearest the centre; u(n)/du; w
     int direct;       // no recurrence: see the staging
 };
@@ -173,6 +191,7 @@ __global__ void __launch_bounds__(kSincBlock, 4) sincsq_uniform_kernel(
 #pragma unroll
     for (int m = 0; m < BINS; ++m) acc[m] = 0.0;
     const double inv_pi = 1.0 / kPi, inv_dE = 1.0 / dE;
+    const double first = (double)bin0, last = (double)((bin0 + kWindow < n_E ? bin0 + kWindow : n_E) - 1);
     // the coefficients in scalar registers, from which an FMA reads them directly
     double sin_r[7], cos_r[8];
 #pragma unroll
@@ -202,18 +221,25 @@ __global__ void __launch_bounds__(kSincBlock, 4) sincsq_uniform_kernel(
             o.du = al * dE;
             sincospi(o.du - 2.0 * rint(0.5 * o.du), &o.sd, &o.cd);
             const double inv_du = rcp_nr(o.du);
-            o.q = inv_pi * inv_du;
+            o.q = inv_pi * (1.0 - kRcpMean) * inv_du;
             const double n = rint((er - E0) * inv_dE), u = fma(n, o.du, o.u0);
             o.nf = (float)(n - (double)bin0);
             o.f = (float)(u * inv_du);
             o.w = wl;
-            // At the centre sine and distance vanish together.  The sine there is
-            // off by up to 1e-13 of the largest of the run, min(1, 8 pi du), and by
-            // the rounding of its phase, 1e-15 du: below 3e-8 of itself unless
-            // |u(n)| is under this line, where every cell is taken on its own
-            // (1 line in 1e4 at most).  So are steps too small to divide by.
-            const double small = 4.0e-6 * fmin(1.0, 25.0 * fabs(o.du)) + 4.0e-8 * fabs(o.du);
-            o.direct = !(fabs(o.du) >= 1.0e-250) || !(fabs(u) >= small);
+            // A line with a bin of this window in its central half period takes every
+            // cell on its own: there sine and distance vanish together, and the two
+            // rounded apart would leave 1.05e-7 a cell (root mean square) where one
+            // rounding for both leaves 4.9e-8; elsewhere the stepped cell has 1.05e-7
+            // and the one with a phase 1.2e-7.  Lines narrower than a bin, du >> 1,
+            // are 1 in du of these (5 % of the lines of 5 MeV electrons on 48 eV bins);
+            // those wider than one are all of them.  So are steps too small to divide by.
+            const double nearest = fma(fmin(fmax(n, first), last), o.du, o.u0);
+            o.direct = !(fabs(o.du) >= 1.0e-250) || !(fabs(nearest) >= 0.5);
+            if (!isfinite(fma(first, o.du, o.u0)) || !isfinite(fma(last, o.du, o.u0))) {  // a profile of 1
+                o.u0 = 0.0;
+                o.du = 0.0;
+                o.direct = 1;
+            }
             lines[__popcll(live & ((1ULL << lane) - 1ULL))] = o;
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -230,11 +256,11 @@ __global__ void __launch_bounds__(kSincBlock, 4) sincsq_uniform_kernel(
                 const SincLine &o = lines[j];
                 if (__builtin_amdgcn_readfirstlane(o.direct)) {
                     double k = kb - kMid;
-                    asm volatile("" : "+v"(k));  // keeps the run's bins out of registers outside this rare branch
+                    asm volatile("" : "+v"(k));  // keeps the run's bins out of registers outside this branch
 #pragma unroll
                     for (int m = 0; m < BINS; ++m) {
                         const double u = fma(k + m, o.du, o.u0);
-                        g[m] = fmaf(o.w, sinc2_cell((float)(u - rint(u)), (float)u), g[m]);
+                        g[m] = fmaf(o.w, sinc2_near((float)(u - rint(u)), (float)u), g[m]);
                     }
                     continue;
                 }
@@ -1174,8 +1200,7 @@ hr_status brem_plan(int64_t n_seg, int64_t n_E, BremPlan &P) {
 // of `per` lines, 64 where that leaves every resident wave four, fewer on small
 // inputs so that all of them work.  Dead lines come in runs, so where chunks
 // abound four times the resident blocks are launched to even the waves out
-// (2.7e6 lines on 1024 bins, the weight still on the sines: 448 us resident, 402
-// so; 1.8e5 lines lose 20 us).
+// (2.7e6 lines on 1024 bins: 464 us resident, 451 so, and 9 more in the row sum).
 struct SincPlan {
     int bins = 16, per = kSincChunk;
     int64_t gx = 1, windows = 1;
