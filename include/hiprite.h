@@ -433,7 +433,7 @@ hr_status hr_sincsq_workspace_bytes(const hr_sincsq_args *args, size_t *bytes);
  * ends (args->ws is ignored).  No counterpart in the reference: it is for
  * callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops).  Sizes whose partials exceed the array are refused
- * with HR_ERR_INVALID (at most about 1M bins on a 256-CU device).  Every call
+ * with HR_ERR_INVALID (beyond 2^21 bins on a 256-CU device).  Every call
  * on one device shares the array: calls that overlap on one device (two
  * streams, or two host threads) race.  Results equal hr_sincsq_reduce's bit
  * for bit. */

@@ -1219,10 +1219,12 @@ hr_status sinc_plan(int64_t n_lines, int64_t n_E, SincPlan &P) {
             P.windows = win;
         }
     }
-    int64_t room = 4 * (int64_t)cu / (P.windows > 0 ? P.windows : 1);
-    room = room < 1 ? 1 : room;
+    const int64_t resident = 4 * (int64_t)cu, windows = P.windows > 0 ? P.windows : 1;
+    int64_t room = resident < windows ? 1 : resident / windows;
     while (P.per > 8 && n_lines < room * kSincWaves * P.per * 4) P.per /= 2;
-    if (P.per == kSincChunk) room *= 4;
+    // (a grid of more windows than blocks keeps one row: four would pass the bound of
+    // hr_sincsq_reduce_static)
+    if (P.per == kSincChunk) room = 4 * resident < windows ? 1 : 4 * resident / windows;
     const int64_t chunks = (n_lines + P.per - 1) / P.per;
     const int64_t want = (chunks + kSincWaves - 1) / kSincWaves;
     P.gx = want < room ? (want > 0 ? want : 1) : room;

@@ -141,3 +141,29 @@ def test_lines_without_a_finite_phase_have_a_profile_of_one(device):
     a = np.array([0.1, np.inf, 0.1, np.nan])
     w = np.array([1.0, 2.0, 4.0, 8.0], dtype=np.float32)
     np.testing.assert_array_equal(_reduce(E_r, a, w, 1000.0, 47.9, 300, device), 15.0)
+
+
+@pytest.mark.parametrize("n_E", [1_048_577, 1_500_000, 2_097_152])
+def test_static_scratch_takes_grids_of_two_million_bins(device, n_E):
+    """The static array holds the partial rows of every grid up to 2^21 bins, at line
+    counts that take chunks of 64 (1,024 lines and more where windows outnumber blocks)."""
+    import torch
+
+    from pyrite_amd import _lib
+
+    rng = np.random.default_rng(n_E)
+    E0, dE, n = 1000.0, 0.05, 1100
+    E_r, a, w = E0 + dE * n_E * rng.random(n), 3.0 * rng.random(n) / dE, rng.random(n).astype(np.float32)
+    t = [torch.as_tensor(v, device=device) for v in (E_r, a, w)]
+    out = torch.zeros(n_E, dtype=torch.float64, device=device)
+    args = _lib.SincsqArgs()
+    args.n_lines, args.E_r, args.a, args.w = n, *(v.data_ptr() for v in t)
+    args.n_E, args.E_grid, args.uniform, args.E0, args.dE, args.out = n_E, None, 1, E0, dE, out.data_ptr()
+    _lib.check(_lib.load().hr_sincsq_reduce_static(C.byref(args), C.c_void_p(torch.cuda.current_stream().cuda_stream)),
+               "hr_sincsq_reduce_static")
+    got = out.cpu().numpy()
+    np.testing.assert_allclose(got, _reduce(E_r, a, w, E0, dE, n_E, device), rtol=0, atol=1e-14)
+    k = np.unique(np.concatenate([[0, n_E - 1], rng.integers(0, n_E, 300), np.rint((E_r[:100] - E0) / dE).astype(int)]))
+    k = k[k < n_E]
+    want = (w.astype(float)[:, None] * np.sinc((a / np.pi)[:, None] * (E0 + dE * k - E_r[:, None])) ** 2).sum(0)
+    assert np.all(np.abs(got[k] - want) <= 1e-6 * want + 1e-9)
