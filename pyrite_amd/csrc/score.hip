@@ -410,8 +410,8 @@ constexpr double kLn2d = 0.6931471805599453;
 //
 // So the rows are first ordered by class, those that add nothing dropped (a stable
 // counting sort: the order, and with it the sum, is fixed), and the polynomials of
-// the classes that occur are laid out, 30 us in three launches, from kBremSortCells
-// cells on.  Before (one order, four tiles of 128 rows to a block) and now, us:
+// the classes that occur are laid out, 30 us in three launches, where there is enough
+// to gain (brem_plan).  Before (one order, four tiles of 128 rows to a block) and now, us:
 // 150,000 rows of 0.5..5 MeV x 1,024 bins 234 -> 143 (222 unordered), 150,001 of
 // 5 keV..10 MeV x 2,000 with a quarter dead 271 -> 230 (268), 1e6 of 5 keV..5 MeV x
 // 1,024 990 -> 720 (976); below the limit 60,000 x 1,024 93 -> 79 (82 ordered),
@@ -419,7 +419,7 @@ constexpr double kLn2d = 0.6931471805599453;
 constexpr int kBremStage = 128;  // rows staged at a time
 constexpr int kBremDeg = 6, kBremNodes = kBremDeg + 1;
 constexpr double kBremReach = 8.0;
-constexpr int64_t kBremSortCells = 100'000'000;
+constexpr int64_t kBremSortCells = 100'000'000, kBremSortRows = 20'480, kBremSortBins = 65'536;
 
 // Chebyshev points x_i = cos(pi (2i + 1)/14) of [-1, 1] and, row j, the weights of
 // the values there in coefficient j of the polynomial through them.
@@ -1155,7 +1155,13 @@ hr_status dense_plan(int64_t n_items, int64_t tile, int64_t n_E, DensePlan &P) {
 // Launch shape and workspace of the brem reduction: bins per thread to the grid
 // (a 201-bin grid takes one, not four), tiles of a power of two rows, at least 32,
 // that make up to 16 blocks per CU (rows below the bins' energies cost less than
-// others, direct ones more), and the class order where it pays.
+// others, direct ones more), and the class order where it pays: from 1e8 cells, whose
+// direct evaluation takes 120 us, and from 160 rows a class on, since a class of a bin
+// costs as much as the polynomial saves in some 150 rows (20,480 rows x 4,883 bins of
+// 5 keV..10 MeV 141 us against 122 cell by cell, 163 with the tiles before; of
+// 0.5..5 MeV 124 against 137; 2,048 x 48,829 458 and 341 against 130).  The
+// polynomials and the classes' own rows take 4.6 kB a bin, 300 MB at kBremSortBins,
+// beyond which rows stay as they lie in the 32 MB of the direct route.
 constexpr int kBremWaves = 512;  // of the sort, at most
 struct BremPlan {
     int bins = 4;
@@ -1175,8 +1181,9 @@ hr_status brem_plan(int64_t n_seg, int64_t n_E, BremPlan &P) {
     // sizes at their bounds, so that a workspace serves fewer rows too
     const bool some = n_seg > 0 && n_E > 0;
     int64_t rows_max = (n_seg + 31) / 32 < room ? (n_seg + 31) / 32 : room;
-    // row indices of the order are 32-bit, and so is the laying grid
-    if (some && n_seg <= INT32_MAX && n_E <= (1 << 24) && n_seg >= kBremSortCells / n_E) {
+    // row indices of the order are 32-bit
+    if (some && n_seg >= kBremSortRows && n_seg <= INT32_MAX && n_E <= kBremSortBins &&
+        n_seg >= kBremSortCells / n_E) {
         P.per = (n_seg + kBremWaves - 1) / kBremWaves;
         P.per = P.per < 256 ? 256 : (P.per + 63) / 64 * 64;
         P.waves = (n_seg + P.per - 1) / P.per;
