@@ -19,9 +19,12 @@ namespace hr {
 namespace {
 
 constexpr int kQueueMaxCfg = 1024;
-// Configurations whose element constants a block keeps in LDS (52 KB: two
-// 256-lane blocks share a CU's 160 KB); later ones and stacks build them per row.
+// Configurations whose element constants a block keeps in LDS (56 KB, 64 with the
+// offsets: two 256-lane blocks share a CU's 160 KB); later ones and stacks build them
+// per row.
 constexpr int kQueueEl = 512;
+static_assert(2 * (kQueueEl * sizeof(ElConst) + (kQueueMaxCfg + 1) * sizeof(int64_t)) <= 160 * 1024,
+              "two blocks to a CU");
 constexpr int kTally = HR_QUEUE_TALLY;
 
 __device__ __forceinline__ int find_config(const int64_t *__restrict__ off, int n_cfg, int64_t i) {

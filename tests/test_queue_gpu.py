@@ -105,3 +105,20 @@ def test_autotuner_picks_a_timed_candidate(device, tmp_path):
     rec2 = TransportQueue(_cases(), device).autotune(fraction=0.5, blocks=(64, 256), claims=(1, 4),
                                                      cache=tmp_path / "tune.json")
     assert rec2["best"] == rec["best"]
+
+
+def test_element_constants_beyond_the_table_and_of_compounds(device):
+    """Configurations from the 513th on, and layers of several elements, build the
+    straggling constants per row instead of reading the block's table."""
+    from pyrite_amd.queue import QueueCase, TransportQueue
+
+    film = [("Si", 0.025), ("C", 0.05)]
+    cases = [QueueCase(Ne=2 + i % 3, thickness_ang=3.0e3, E0_keV=8.0 + (i % 7), material=("Si", "W")[i % 2], seed=i + 1)
+             for i in range(515)]
+    cases[0] = QueueCase(Ne=200, thickness_ang=2.0e4, E0_keV=40.0, material="Si", composition=film, seed=9)
+    for i, m in ((511, "Ge"), (512, "W"), (513, "graphite")):
+        cases[i] = QueueCase(Ne=150, thickness_ang=1.0e4, E0_keV=30.0, material=m, seed=i)
+    cases[514] = QueueCase(Ne=100, thickness_ang=2.0e4, E0_keV=40.0, material="Si", composition=film, seed=10)
+    got = TransportQueue(cases, device).run().cpu().numpy()
+    for i in (0, 1, 2, 510, 511, 512, 513, 514):
+        np.testing.assert_array_equal(got[i], _per_config_tally(cases[i], device), err_msg=f"config {i}")
