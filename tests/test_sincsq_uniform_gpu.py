@@ -167,3 +167,49 @@ def test_static_scratch_takes_grids_of_two_million_bins(device, n_E):
     k = k[k < n_E]
     want = (w.astype(float)[:, None] * np.sinc((a / np.pi)[:, None] * (E0 + dE * k - E_r[:, None])) ** 2).sum(0)
     assert np.all(np.abs(got[k] - want) <= 1e-6 * want + 1e-9)
+
+
+# Lines that make a wave's chunk 16, 32 and 64 on 256 CUs and one window of bins (8 below the
+# first): 16 waves a CU with four chunks each, 256 x 16 x 4 x the chunk.  Chunks of 64 also take
+# four times the resident blocks.
+CHUNK_LINES = {16: 262_144, 32: 524_288, 64: 1_048_576}
+
+
+@pytest.mark.parametrize("n_E", [61, 777])
+@pytest.mark.parametrize("chunk", list(CHUNK_LINES))
+def test_long_chunks_match_fp64(device, chunk, n_E):
+    """Ragged last chunks, runs of lines without weight as long as several chunks, and eighths
+    that are alive, dead and partly dead, against torch in FP64."""
+    import torch
+
+    from pyrite_amd import _lib
+
+    rng = np.random.default_rng([chunk, n_E])
+    n, E0, dE = CHUNK_LINES[chunk] + 77, 1000.0, 47.9
+    E_r, a, w = _lines(rng, n, E0, dE, n_E)
+    w[:chunk * 8] = rng.uniform(0.5, 1.0, chunk * 8)          # every eighth alive
+    w[chunk * 8:chunk * 24] = 0.0                              # whole chunks dead
+    w[chunk * 24:chunk * 40].reshape(-1, 8)[::3] = 0.0         # every third eighth dead
+    w[chunk * 40:chunk * 56].reshape(-1, 8)[:, 1:7] = 0.0      # eighths with their ends alive
+    dead = np.repeat(rng.random(n // 1000 + 1) < 0.3, 1000)[:n]
+    w[chunk * 56:][dead[chunk * 56:]] = 0.0
+    args = _lib.SincsqArgs()
+    args.n_lines, args.n_E, args.uniform, args.E0, args.dE = n, n_E, 1, E0, dE
+    rows = _lib.workspace_bytes("hr_sincsq_workspace_bytes", C.byref(args)) // (8 * n_E)
+    if torch.cuda.get_device_properties(device).multi_processor_count == 256:
+        assert rows == (4096 if chunk == 64 else 1024)
+    got = _reduce(E_r, a, w, E0, dE, n_E, device)
+    t = [torch.as_tensor(v, dtype=torch.float64, device=device) for v in (E_r, a, w)]
+    want, size, envelope = (torch.zeros(n_E, dtype=torch.float64, device=device) for _ in range(3))
+    k = torch.arange(n_E, dtype=torch.float64, device=device)
+    for s in range(0, n, 1 << 16):
+        Er, al, wl = (v[s:s + (1 << 16), None] for v in t)
+        al = al / np.pi
+        u = k * (al * dE) + al * (E0 - Er)
+        r = u - torch.round(u)
+        cell = torch.where(u == 0.0, 1.0, torch.sin(np.pi * r) / (np.pi * torch.where(u == 0.0, 1.0, u))) ** 2
+        want += (wl * cell).sum(0)
+        size += (wl.abs() * cell).sum(0)
+        envelope += (wl.abs() / torch.clamp((np.pi * u) ** 2, min=1.0)).sum(0)
+    bound = (1e-6 * size + 1e-9 * envelope + 1e-15).cpu().numpy()
+    assert np.all(np.abs(got - want.cpu().numpy()) <= bound), float(np.max(np.abs(got - want.cpu().numpy()) / bound))
