@@ -118,7 +118,6 @@ __device__ __forceinline__ float sinc2_near(float r, float uf) {
 }
 
 constexpr int kRedThreads = 256;
-constexpr int kLineTile = 256;  // lines staged in LDS per step
 constexpr int kSincGroup = 4;   // cells summed in FP32 before each FP64 add (all terms >= 0)
 
 // ---- dense sum over a uniform grid E_k = E0 + k dE
@@ -307,9 +306,9 @@ __global__ void __launch_bounds__(kSincBlock, 4) sincsq_uniform_kernel(
 // evaluates as many of a thread's bins as reach the grid (777 bins: 13 of 16 runs
 // of 64), and a block's lines are short tiles from all over the input, since lines
 // without weight come in runs.  Bound by vector instructions, some 80 SIMD cycles a
-// cell.  Reduction before (four bins each, 256 lines in a row) and now: 150,000
-// live lines of 320,000 x 777 bins 126 -> 101 us, x 257 bins 124 -> 55, x 1,024 122 ->
-// 117, 38,000 of 80,000 x 201 bins 66 -> 31.
+// cell.  The call before (four bins each, 256 lines in a row) and now: 150,000 live
+// lines of 320,000 x 777 bins 130 -> 98 us, x 300 128 -> 49, x 1,024 129 -> 111, 38,000
+// of 80,000 x 201 bins 75 -> 26, of 1,200 x 777 51 -> 22 (53 with a block to 256 lines).
 constexpr int kGeneralTile = 64;
 template <int BINS>
 __global__ void __launch_bounds__(kRedThreads) sincsq_general_kernel(
@@ -1135,20 +1134,20 @@ int64_t line_blocks(int cu, int64_t n_tiles, int64_t bin_tiles) {
 
 constexpr int kDenseBins = 4;  // bins per thread of the dense reducers
 
-// Launch shape and workspace bytes of a dense reducer over n_items items in
-// tiles of `tile`, on a grid of n_E bins, for the current device.
+// Launch shape and workspace bytes of the general reduction of n_lines lines on
+// n_E bins, for the current device.
 struct DensePlan {
     int64_t gx = 0, bin_tiles = 0;
     size_t bytes = 0;
 };
-hr_status dense_plan(int64_t n_items, int64_t tile, int64_t n_E, DensePlan &P) {
+hr_status dense_plan(int64_t n_lines, int64_t n_E, DensePlan &P) {
     int cu = 0;
     hr_status st = device_cu(cu);
     if (st != HR_OK) return st;
     P.bin_tiles = (n_E + kRedThreads * kDenseBins - 1) / (kRedThreads * kDenseBins);
-    const int64_t n_tiles = (n_items + tile - 1) / tile;
+    const int64_t n_tiles = (n_lines + kGeneralTile - 1) / kGeneralTile;
     P.gx = line_blocks(cu, n_tiles, P.bin_tiles);
-    P.bytes = (n_items == 0 || n_E == 0) ? 0 : partial_bytes(P.gx, n_E);
+    P.bytes = (n_lines == 0 || n_E == 0) ? 0 : partial_bytes(P.gx, n_E);
     return HR_OK;
 }
 
@@ -1252,7 +1251,7 @@ hr_status sinc_bytes(const hr_sincsq_args &p, size_t &bytes) {
         return st;
     }
     DensePlan P;
-    hr_status st = dense_plan(p.n_lines, kLineTile, p.n_E, P);
+    hr_status st = dense_plan(p.n_lines, p.n_E, P);
     bytes = P.bytes;
     return st;
 }
@@ -1331,7 +1330,7 @@ extern "C" hr_status hr_sincsq_reduce(const hr_sincsq_args *args, void *stream) 
         return row_sum((const double *)ws, P.gx, p.n_E, p.out, s);
     }
     DensePlan P;
-    hr_status st = dense_plan(p.n_lines, kLineTile, p.n_E, P);
+    hr_status st = dense_plan(p.n_lines, p.n_E, P);
     if (st != HR_OK) return st;
     HR_REQUIRE_WS(p.ws, P.bytes, "hr_sincsq_reduce");
     const dim3 grid((unsigned)P.gx, (unsigned)P.bin_tiles);
@@ -1378,7 +1377,7 @@ extern "C" hr_status hr_sincsq_reduce_static(const hr_sincsq_args *args, void *s
     // the sizes taken are those whose general-grid partials (and 64 more rows) fit, whatever the grid
     DensePlan P;
     size_t need = 0;
-    hr_status st = dense_plan(args->n_lines, kLineTile, args->n_E, P);
+    hr_status st = dense_plan(args->n_lines, args->n_E, P);
     if (st == HR_OK) st = sinc_bytes(*args, need);
     if (st != HR_OK) return st;
     const size_t limit = partial_bytes(P.gx + (P.gx < 64 ? P.gx : 64), args->n_E);

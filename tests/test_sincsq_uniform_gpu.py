@@ -1,4 +1,4 @@
-"""The uniform-grid sinc^2 reduction at the edges of its windows, runs and chunks (GPU).
+"""The sinc^2 reductions at the edges of their windows, runs, chunks and tiles (GPU).
 
 Against the FP64 profile in numpy.  The bound: a cell's factor x carries the
 rounding of the sine, the two of the distance, the reciprocal's ulp and the
@@ -213,3 +213,37 @@ def test_long_chunks_match_fp64(device, chunk, n_E):
         envelope += (wl.abs() / torch.clamp((np.pi * u) ** 2, min=1.0)).sum(0)
     bound = (1e-6 * size + 1e-9 * envelope + 1e-15).cpu().numpy()
     assert np.all(np.abs(got - want.cpu().numpy()) <= bound), float(np.max(np.abs(got - want.cpu().numpy()) / bound))
+
+
+@pytest.mark.parametrize("n_E", [2, 63, 65, 256, 257, 700, 1024, 1025])
+@pytest.mark.parametrize("n", [1, 63, 65, 1200, 140_000])
+def test_general_grid_matches_fp64(device, n, n_E):
+    """A grid without a step at the edges of tiles of 64 lines, runs of 64 bins and windows of
+    1,024, one block to a tile until 8 a CU share them."""
+    import torch
+
+    from pyrite_amd import _lib
+
+    rng = np.random.default_rng([n, n_E])
+    grid = np.geomspace(1000.0, 50_000.0, n_E)
+    E_r, a, w = _lines(rng, n, 1000.0, 49_000.0 / n_E, n_E)
+    t = [torch.as_tensor(v, device=device) for v in (E_r, a, w, grid)]
+    out = torch.zeros(n_E, dtype=torch.float64, device=device)
+    args = _lib.SincsqArgs()
+    args.n_lines, args.E_r, args.a, args.w = n, *(v.data_ptr() for v in t[:3])
+    args.n_E, args.E_grid, args.uniform, args.out = n_E, t[3].data_ptr(), 0, out.data_ptr()
+    need = _lib.workspace_bytes("hr_sincsq_workspace_bytes", C.byref(args))
+    blocks = 8 * torch.cuda.get_device_properties(device).multi_processor_count // ((n_E + 1023) // 1024)
+    assert need == 8 * n_E * min(blocks, (n + 63) // 64)
+    args.ws = _lib.DeviceScratch(device).get(need)
+    _lib.check(_lib.load().hr_sincsq_reduce(C.byref(args), C.c_void_p(torch.cuda.current_stream().cuda_stream)),
+               "hr_sincsq_reduce")
+    want, size = (torch.zeros(n_E, dtype=torch.float64, device=device) for _ in range(2))
+    for s in range(0, n, 1 << 15):
+        Er, al, wl = (v[s:s + (1 << 15), None].double() for v in t[:3])
+        u = al / np.pi * (t[3] - Er)
+        cell = torch.where(u == 0.0, 1.0,
+                           torch.sin(np.pi * (u - torch.round(u))) / (np.pi * torch.where(u == 0.0, 1.0, u))) ** 2
+        want += (wl * cell).sum(0)
+        size += (wl.abs() * cell).sum(0)
+    assert bool(torch.all((out - want).abs() <= 1.0e-6 * size + 1.0e-15))
