@@ -533,8 +533,8 @@ def main():
     ms = [ev[0].elapsed_time(ev[1]) for ev, _ in pipe.lines.events] or [float("nan")]
     cells = live_cells(pipe, args.steps, len(ms))  # live (nonzero-weight) lines x bins of the timed launches
     avg_ms = sum(ms) / len(ms)
-    flops_per_launch = roofline.SINC_CELL_OPS * cells / len(ms)
-    achieved = flops_per_launch / (avg_ms * 1e-3) / 1e12
+    cells_per_s = cells / len(ms) / (avg_ms * 1e-3)
+    achieved = roofline.SINC_STEPPED_CELL_OPS * cells_per_s / 1e12  # what the kernel spends
     line_bytes = 20  # E_r f64 + a f64 + w f32 per line, read once per launch
     n_E = cfg.n_bins
     lines_per_launch = cells / len(ms) / n_E
@@ -570,7 +570,11 @@ def main():
             "traffic": SINC_TRAFFIC_BYTES if (args.ne, args.n_side, args.line_route) == (100_000, 3, "dense") else None,
             "traffic_source": "rocprofv3 --pmc FETCH_SIZE (x2.000) and WRITE_SIZE (x1.000), factors from a 1 GiB "
                               "copy; profiles/sincsq_uniform_hopg_5mev_pmc.md",
-            "ops_per_cell": roofline.SINC_CELL_OPS,
+            "ops_per_cell": roofline.SINC_STEPPED_CELL_OPS,
+            # work done by the count of the reference's cell (a sine and a division 20 each):
+            # a rate, not a share of the machine
+            "reference_ops_per_cell": roofline.SINC_CELL_OPS,
+            "reference_rate": roofline.SINC_CELL_OPS * cells_per_s / 1e12,
             "live_cells_per_launch": cells / len(ms),
             "avg_launch_ms": avg_ms,
             "launches": len(ms),

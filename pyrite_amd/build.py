@@ -4,8 +4,10 @@
 for ``--offload-arch=gfx950`` and links ``pyrite_amd/_lib/libhiprite.so``.
 Packed-FP32 instruction selection is disabled on every unit
 (``-target-feature -packed-fp32-ops``).  Units whose arithmetic is compared
-against the FP64 oracle step by step are compiled with ``-ffp-contract=off``
-(the reproducible math mode); the others keep hipcc's default contraction.
+against the FP64 oracle step by step are compiled with ``-ffp-contract=off``: the
+compiler fuses nothing there, and the fused multiply-adds are those that the
+source writes.  The others keep hipcc's default contraction, the work queue among
+them, whose transport step may therefore differ from theirs in the last bit.
 """
 
 from __future__ import annotations
@@ -25,7 +27,7 @@ LIB = LIBDIR / "libhiprite.so"
 BUILD = PKG / "_build"
 
 ARCH = os.environ.get("HIPRITE_ARCH", "gfx950")
-# Units checked step by step against the FP64 oracle: no fused multiply-add.
+# Units checked step by step against the FP64 oracle: no fused multiply-add but the written ones.
 REPRODUCIBLE = {"transport.hip", "vr.hip", "cone.hip"}
 
 

@@ -21,8 +21,9 @@ __device__ __forceinline__ double rcp_nr(double x) {
     return fma(fma(-x, r, 1.0), r, r);
 }
 
-// a/b from r = 1/b: the product and one correction by its exact remainder, the
-// correctly rounded quotient but for rare last-bit ties.
+// a/b from r = 1/b: the product and one correction by its exact remainder (P.
+// Markstein, IBM J. Res. Dev. 34 (1990) 111), the correctly rounded quotient but for
+// rare last-bit ties.
 __device__ __forceinline__ double div_by(double a, double b, double r) {
     const double q = a * r;
     return fma(fma(-q, b, a), r, q);

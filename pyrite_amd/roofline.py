@@ -9,11 +9,16 @@ here so the builder and any reviewer compute the same fraction:
 * an FMA counts as 2 operations.
 
 Per-unit counts (estimates of the reference algorithm, not of these kernels'
-instruction stream):
+instruction stream, but for ``SINC_STEPPED_CELL_OPS``):
 
 * sinc^2 cell, one (line, bin): phase ``a (E - E_r)`` (2), reduction to
   ``[-pi/2, pi/2]`` (2), square and scale (4): 8 FP ops, plus one sin and
   one division -> ``8 + 2*20 = 48`` FP32-equivalent operations;
+* the same cell as the kernel of uniform grids takes it, its sine stepped from the
+  two bins before: the FP64 FMA (2 operations at half the FP32 rate, 4), the
+  conversion (1), the distance in bins (2), its reciprocal (1, one instruction),
+  the ratio, and weight times square added up (1 + 1 + 2) -> 12 operations.  A
+  fraction of the peak counts these; the 48 give a rate of work done;
 * brem cell, one (segment, bin, element): about 25 FP ops plus log, exp, sqrt,
   exp and expm1 of the escape mean -> ``25 + 5*20 = 125``;
 * transport step (LUT, screened Rutherford, midpoint rule, one element, Urban
@@ -32,6 +37,7 @@ TRANSCENDENTAL_FP32 = 20
 TRANSCENDENTAL_FP64 = 40
 
 SINC_CELL_OPS = 8 + 2 * TRANSCENDENTAL_FP32
+SINC_STEPPED_CELL_OPS = 12
 BREM_CELL_OPS = 25 + 5 * TRANSCENDENTAL_FP32
 TRANSPORT_STEP_OPS_FP64 = 90 + 6 * TRANSCENDENTAL_FP64
 LINE_PROLOGUE_OPS_FP64 = 220 + 8 * TRANSCENDENTAL_FP64

@@ -190,7 +190,8 @@ class CoherentScorer:
                     n_lines)
 
     def _launch_grouped(self, rec, n_lines, group_start):
-        """The grouped term alone."""
+        """The grouped term alone (``hr_coherent_grouped``, the entry of callers that keep a
+        flat field of their own); ``add_rows`` takes both in one pass."""
         g = _lib.CoherentGroupedArgs()
         self._field_args(g.field, rec, n_lines)
         g.group_start, g.n_groups = group_start.data_ptr(), int(group_start.numel()) - 1
