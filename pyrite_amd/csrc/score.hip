@@ -133,10 +133,10 @@ constexpr int kSincGroup = 4;   // cells summed in FP32 before each FP64 add (al
 // square on its own and FP32 groups end with every eighth line of the input, so that
 // weighted copies add up to the unweighted sum (a weight of 2 is twice the line).
 //
-// VALU bound: about 31 SIMD cycles per cell (FP64, conversions and selects issue
+// VALU bound: about 30 SIMD cycles per cell (FP64, conversions and selects issue
 // in 4, plain FP32 in 2, the reciprocal in 8) against 52 of a cell with its own
 // phase.  2.7e6 lines of 5 MeV electrons (1.47e6 live) on 1024 bins of 48 eV: 600 us
-// with a phase per cell, 451 so (about 40 cycles: staging, the lines taken cell by
+// with a phase per cell, 451 so (about 43 cycles: staging, the lines taken cell by
 // cell, FP64 sums and waves of uneven work make the rest).  Lines wider than a bin
 // are all taken cell by cell: 1e6 of them on 1024 bins 523 us before, 513 so.
 constexpr int kSincWaves = 4;     // waves per block, each with its own lines
@@ -305,8 +305,9 @@ __global__ void __launch_bounds__(kSincBlock, 4) sincsq_uniform_kernel(
 // degenerate uniform grid E0 + k dE whose step is zero or not finite).  A wave
 // evaluates as many of a thread's bins as reach the grid (777 bins: 13 of 16 runs
 // of 64), and a block's lines are short tiles from all over the input, since lines
-// without weight come in runs.  Bound by vector instructions, some 80 SIMD cycles a
-// cell.  The call before (four bins each, 256 lines in a row) and now: 150,000 live
+// without weight come in runs.  Bound by vector instructions, 22 a cell, some 60 SIMD
+// cycles by their issue (65 measured where most lines live, 114 where a third does).
+// The call before (four bins each, 256 lines in a row) and now: 150,000 live
 // lines of 320,000 x 777 bins 130 -> 98 us, x 300 128 -> 49, x 1,024 129 -> 111, 38,000
 // of 80,000 x 201 bins 75 -> 26, of 1,200 x 777 51 -> 22 (53 with a block to 256 lines).
 constexpr int kGeneralTile = 64;
@@ -399,10 +400,10 @@ constexpr double kLn2d = 0.6931471805599453;
 //
 // A cell is A g(T, k) e(path, mu_k): the segment's length and weight, the Born
 // cross section with its Elwert factors, which depend on the energy and the bin
-// alone, and the mean escape.  The kernel is bound by vector instructions, 40 a
+// alone, and the mean escape.  The kernel is bound by vector instructions, 39 a
 // cell.  g is smooth in T away from the spectral tip, so rows of one energy class,
 // an eighth of an octave, can take it as a polynomial of degree 6 per bin, through
-// seven Chebyshev points of the class evaluated in FP64: 23 instructions a cell.
+// seven Chebyshev points of the class evaluated in FP64: 22 instructions a cell.
 // The nearest singularity is T = k: a class c +- h with (c - k) >= 8 h interpolates
 // to 16^-7 = 4e-9 of g; closer classes (energies below about twice the bin's)
 // evaluate every cell.
